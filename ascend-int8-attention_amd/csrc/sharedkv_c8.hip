@@ -38,6 +38,8 @@
 // large decode batches; any head count, no explicit slots) run c8_rows instead:
 // two four-wave work-groups per CU with one tile buffer each, each taking
 // rows in turn, so that one row's tile chain fills the other's waits.
+// C128 and window-only prefill chunks run c8_chunk: one row per wave, eight
+// neighbouring rows sharing their KV tiles.
 // Integer partials are exact, so any assignment of keys to lanes gives the
 // reference's integers; the FP32 sequence below is kept in the reference's
 // order with contraction disabled.
@@ -465,14 +467,14 @@ __device__ __forceinline__ void fold_row(const __amdgpu_buffer_rsrc_t states, in
 // written.  Above eight heads the Q and P residual codes are zero
 // (reference.py:221-222: residual quantization only for <= 8 heads), which
 // leaves every other operation as it is.  Without ANYH, heads == 8.
+// The work of one work-group: item `item` of the launch's `items`.
 template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT>
-__global__ void __launch_bounds__(THREADS, 1)   // one work-group per CU: the 128 KiB tile ring fills the LDS
-c8_attention(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint64_t cmp_indices,
-             const uint32_t batch_arg, const uint32_t topk_arg, const uint32_t heads_arg, const uint32_t splits,
-             const uint32_t rows_arg, const uint32_t grid, const SharedKVArgs p, const SharedKVDebug dbg,
-             const uint32_t fused)
+__device__ __forceinline__ void
+attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint64_t cmp_indices,
+               const uint32_t batch_arg, const uint32_t topk_arg, const uint32_t heads_arg, const uint32_t splits,
+               const uint32_t rows_arg, const uint32_t grid, const SharedKVArgs &p, const SharedKVDebug &dbg,
+               const uint32_t fused, const uint32_t items)
 {
-    __shared__ Shared s;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
 
     // XCD-aware order: consecutive work items (the partitions of one row,
@@ -480,7 +482,6 @@ c8_attention(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base
     // items [x G / 8, (x + 1) G / 8).
     const uint32_t G = grid;
     const uint32_t item = (blockIdx.x & 7u) * (G >> 3) + (blockIdx.x >> 3);
-    const uint32_t items = rows_arg * splits;
     if (item >= items) return;
     const int H = ANYH ? (int)heads_arg : HEADS;                 // heads of a query token
     const int HG = ANYH ? (H + HEADS - 1) / HEADS : 1;           // groups of eight
@@ -1476,6 +1477,19 @@ c8_attention(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base
     } else {
         run_row(std::integral_constant<bool, false>{});
     }
+}
+
+template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT>
+__global__ void __launch_bounds__(THREADS, 1)   // one work-group per CU: the 128 KiB tile ring fills the LDS
+c8_attention(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint64_t cmp_indices,
+             const uint32_t batch_arg, const uint32_t topk_arg, const uint32_t heads_arg, const uint32_t splits,
+             const uint32_t rows_arg, const uint32_t grid, const SharedKVArgs p, const SharedKVDebug dbg,
+             const uint32_t fused)
+{
+    __shared__ Shared s;
+    attention_item<RATIO, DEBUG, SLOTS, ANYH, STREAM, JOINT>(s, cu_q, seq_lens, q_base, cmp_indices, batch_arg, topk_arg,
+                                                             heads_arg, splits, rows_arg, grid, p, dbg, fused,
+                                                             rows_arg * splits);
 }
 
 // Partition merge as a second launch (merge mode 1): one 512-thread group
@@ -2766,6 +2780,785 @@ c8_pairs(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
                       H);
 }
 
+// ---- c8_chunk: prefill chunks whose neighbouring query rows share their KV rows ----
+// One-partition C128 and window-only launches of many rows.  One work-group
+// per row (c8_attention) or one row per four waves (c8_rows) copies every
+// row's KV again and sends every tile through three or four work-group
+// barriers; on these launches those chains and the row set-up bound the time,
+// not the copies.  Here a query row (token, eight heads) belongs to one wave,
+// whose chain QK -> maximum -> exponentials and P codes -> PV crosses no
+// barrier, and the eight rows of a work-group, neighbours in the launch, share
+// every KV tile: the union of their windows (at most 135 rows) and the
+// compressed tiles, which start at the same rows for every token of a request,
+// are copied to LDS once for all eight.
+//   Q codes    a wave encodes its row in registers, straight in the MFMA A
+//              layout: lanes n and n ^ 1 hold the two halves of a head's
+//              16-channel chunks and exchange code against residual by DPP
+//   K/V tiles  row u of a tile lies at u * 512 with its 16-byte chunks
+//              XOR-swizzled by u & 15: any 16 consecutive rows, at any
+//              alignment (the rows' windows are shifted against each other),
+//              hit distinct banks in QK's reads, and two neighbouring 8-row
+//              groups do in PV's
+//   P codes    key-major (16 bytes a key, one 32-bit write per lane and key
+//              block), read back transposed for the MFMA A operand
+//   output     through LDS, so that it leaves in whole 1 KiB heads
+// Bound by the FP32 sequence (about 1250 VALU instructions a wave and tile,
+// 4.2 us for the two waves of a SIMD) and the LDS reads (1 MiB a tile and
+// work-group, 3.4 us), which overlap only in part: a tile takes about 6 us, a
+// window-only octet about 15.  Measured on MI355X, before -> after: B = 1 x
+// T = 2048, C128 at 8 K / 32 K / 128 K context 62 / 79 / 160 -> 27 / 33 / 69
+// us, window-only 26 -> 17; T = 4096 C128 at 32 K 156 -> 62, window-only
+// 48 -> 32.
+typedef __attribute__((address_space(3))) v4i lds_v4i;
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+constexpr int CHUNK_ROWS = 8;                        // query rows of a work-group (one per wave)
+constexpr int CHUNK_UNION = N + CHUNK_ROWS;          // window rows of an octet (135 at most), in pairs
+constexpr int OUT_STRIDE = 2 * D + 32;               // LDS row stride of a head's BF16 output
+
+struct alignas(16) ChunkShared {
+    float scale[2][D];                     // channel scales of the window / compressed cache
+    int8_t bad[2][CHUNK_ROWS];             // per wave: some window row it copied lies on no readable page
+    int8_t window_ok[2][CHUNK_UNION];      // union rows on a readable page
+    int8_t p[CHUNK_ROWS][N * 16];          // P codes of each wave's row [key][MFMA row]
+    alignas(16) int8_t buf[2][CHUNK_UNION * D];   // window unions, compressed tiles, output staging
+};
+static_assert(sizeof(ChunkShared) <= 160 * 1024, "one work-group per CU");
+static_assert(CHUNK_ROWS * HEADS * OUT_STRIDE <= CHUNK_UNION * D, "output staging fits one buffer");
+
+// x rounded to the nearest even integer sits in the low bits of x + MAGIC
+// (|x| < 2^22), so the low byte of the sum is the INT8 code.
+constexpr float MAGIC = 12582912.0f;
+__device__ __forceinline__ uint32_t low_bytes(float a, float b, float c, float d)
+{
+    const uint32_t ab = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x0c0c0400u);
+    const uint32_t cd = __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(c), 0x04000c0cu);
+    return ab | cd;
+}
+
+// num / den, correctly rounded, from the correctly rounded reciprocal r of
+// den: the FMA residual of the product corrects it (Markstein, 1990; den is
+// a softmax denominator, so no operand is subnormal).
+__device__ __forceinline__ float div_by(float num, float den, float r)
+{
+    const float q = num * r;
+    // An infinite quotient's residual is NaN; the median turns that into a
+    // finite number, which leaves the infinity as it is.
+    const float e = __builtin_amdgcn_fmed3f(__builtin_fmaf(-q, den, num), -3.0e38f, 3.0e38f);
+    return __builtin_fmaf(e, r, q);
+}
+
+// LDS DMA of 16 bytes per lane from a scalar base and a 32-bit lane offset.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void dma16_at(uint64_t base, uint32_t offset, uint32_t lds)
+{
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(offset), "s"(base), "s"(lds) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+template <int RATIO, bool ANYH>
+__global__ void __launch_bounds__(THREADS, 1)
+c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint32_t batch_arg,
+         const uint32_t rows_arg, const uint32_t grid, const uint32_t heads_arg, const SharedKVArgs p,
+         const uint32_t fused)
+{
+    static_assert(RATIO == 1 || RATIO == 128, "window-only and C128 launches");
+    __shared__ alignas(16) uint8_t lds[sizeof(ChunkShared) > sizeof(Shared) ? sizeof(ChunkShared) : sizeof(Shared)];
+    ChunkShared &s = *reinterpret_cast<ChunkShared *>(lds);
+    const int tid = threadIdx.x;
+    const int wave = uni(tid >> 6);
+    const __attribute__((address_space(1))) int32_t *cu = gptr<int32_t>(cu_q);
+    const __attribute__((address_space(1))) int32_t *lens = gptr<int32_t>(seq_lens);
+    // SIMD i runs waves i and i + 4.  The first at raised priority: it runs
+    // ahead, so that one wave's VALU phases meet the other's LDS and MFMA ones.
+    if (wave < 4) __builtin_amdgcn_s_setprio(2);
+    const int batch_n = (int)batch_arg;
+    const int H = ANYH ? (int)heads_arg : HEADS;                 // heads of a query token
+    const int HG = ANYH ? (H + HEADS - 1) / HEADS : 1;           // groups of eight
+    const bool resid = !ANYH || H <= HEADS;
+    const int rows_cap = (int)rows_arg;
+    // Every wave holds the metadata of the first 64 requests, request b in
+    // lane b, and searches them with ballots.
+    const int mine_b = (tid & 63) < batch_n ? (tid & 63) : batch_n - 1;
+    const int my_cu0 = cu[mine_b], my_cu1 = cu[mine_b + 1], my_len = lens[mine_b];
+    const f32x2 scale_pair = *gptr<f32x2>(((tid >> 8) && RATIO != 1 ? p.cmpScale : p.oriScale) + (uint64_t)((tid & 255) * 2) * 4);
+
+    // Work: octet o holds rows 8 o .. 8 o + 7 of the launch; XCD x takes a
+    // contiguous eighth of them.
+    const int x = (int)(blockIdx.x & 7u), slot = (int)(blockIdx.x >> 3), per_xcd = (int)(grid >> 3);
+    int octets = (rows_cap + CHUNK_ROWS - 1) / CHUNK_ROWS;
+    auto first_octet = [&](int xcd) { return (int)((int64_t)xcd * octets / 8); };
+    int o = first_octet(x) + slot;
+    // The wave's row of the octet: token t, heads hbase .. hbase + hlive - 1;
+    // its Q (head n / 2, channels 64 j + 16 g + 8 (n & 1) and up) and sinks.
+    int t, hbase, hlive, stop;
+    v4i qraw[8];
+    float sink[2];
+    auto load_row = [&]() {
+        const int row = CHUNK_ROWS * o + wave;
+        t = row < rows_cap ? (ANYH ? row / HG : row) : INT32_MAX;
+        hbase = ANYH ? HEADS * (row % HG) : 0;
+        hlive = ANYH ? (H - hbase < HEADS ? H - hbase : HEADS) : HEADS;
+        const int last = CHUNK_ROWS * o + CHUNK_ROWS < rows_cap ? CHUNK_ROWS * o + CHUNK_ROWS - 1 : rows_cap - 1;
+        stop = (ANYH ? last / HG : last) + 1;
+        int lane = tid & 63;
+        asm volatile("" : "+v"(lane));
+        const int g = lane >> 4, n = lane & 15;
+        // Rows past the launch and heads past the last read the first ones
+        // (never written).
+        const int tq = row < rows_cap ? t : 0, hq = row < rows_cap ? hbase : 0;
+        const uint64_t at = q_base + (((uint64_t)tq * H + hq + (!ANYH || (n >> 1) < hlive ? n >> 1 : 0)) * D + 16 * g + 8 * (n & 1)) * 2;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) qraw[j] = __builtin_nontemporal_load(gptr<v4i>(at + 128 * j));
+        const __attribute__((address_space(1))) float *sinks = gptr<float>(p.sinks);
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) sink[hh] = sinks[hq + (!ANYH || 2 * g + hh < hlive ? 2 * g + hh : 0)];
+    };
+    load_row();
+
+    // ---- live shape (attention_impl.h:121-137) ----
+    // The last request with seq_len > 0 and cu_q >= 0 ends the live batch;
+    // its cu_q end bounds the live tokens.
+    int live_batch = 0, end = 0;
+    {
+        const uint64_t there = __ballot((tid & 63) < batch_n && my_len > 0 && my_cu1 >= 0);
+        if (there) {
+            const int b = 63 - __builtin_clzll(there);
+            live_batch = b + 1;
+            end = __builtin_amdgcn_readlane(my_cu1, b);
+        }
+        for (int b0 = 64; b0 < batch_n; b0 += 64) {
+            const int b = b0 + (tid & 63) < batch_n ? b0 + (tid & 63) : batch_n - 1;
+            const int c1 = cu[b + 1];
+            const uint64_t more = __ballot(b == b0 + (tid & 63) && lens[b] > 0 && c1 >= 0);
+            if (more) {
+                live_batch = b0 + 64 - __builtin_clzll(more);
+                end = __builtin_amdgcn_readlane(c1, 63 - __builtin_clzll(more));
+            }
+        }
+    }
+    const int live_tokens = end <= 0 ? 0 : (end < (int)p.tokens ? end : (int)p.tokens);
+    // The request holding `token` (batch < 0: none), as batch, cu[b], cu[b + 1], len.
+    struct Request { int batch, c0, c1, len; };
+    auto find_request = [&](int token) {
+        const uint64_t hit = __ballot((tid & 63) < live_batch && my_cu0 <= token && token < my_cu1);
+        if (hit) {
+            const int b = __builtin_ctzll(hit);
+            return Request{b, __builtin_amdgcn_readlane(my_cu0, b), __builtin_amdgcn_readlane(my_cu1, b),
+                           __builtin_amdgcn_readlane(my_len, b)};
+        }
+        for (int b0 = 64; b0 < live_batch; b0 += 64) {
+            const int b = b0 + (tid & 63) < live_batch ? b0 + (tid & 63) : live_batch - 1;
+            const int c0 = cu[b], c1 = cu[b + 1], len = lens[b];
+            const uint64_t more = __ballot(c0 <= token && token < c1);
+            if (more) {
+                const int at = __builtin_ctzll(more);
+                return Request{b0 + at < live_batch ? b0 + at : live_batch - 1, __builtin_amdgcn_readlane(c0, at),
+                               __builtin_amdgcn_readlane(c1, at), __builtin_amdgcn_readlane(len, at)};
+            }
+        }
+        return Request{-1, 0, 0, 0};
+    };
+    lds_i8 *const buf = (lds_i8 *)s.buf[0], *const pw = (lds_i8 *)s.p[0] + wave * N * 16;
+    auto zero_row = [&](int t, int hbase, int hlive) {
+        const int lane = tid & 63;
+        uint16_t *out = reinterpret_cast<uint16_t *>(p.out) + ((int64_t)t * H + hbase) * D;
+        for (int h = 0; h < hlive; ++h) reinterpret_cast<v4i *>(out)[64 * h + lane] = v4i{0, 0, 0, 0};
+        if (p.lse && lane < hlive) reinterpret_cast<float *>(p.lse)[(int64_t)t * H + hbase + lane] = 0.0f;
+    };
+    if (live_tokens * HG < rows_cap) {
+        // Graph padding: its rows are zero (attention_impl.h:443-460).
+        for (int row = live_tokens * HG + (int)blockIdx.x * CHUNK_ROWS + wave; row < rows_cap; row += (int)grid * CHUNK_ROWS) {
+            const int h = ANYH ? HEADS * (row % HG) : 0;
+            zero_row(ANYH ? row / HG : row, h, ANYH ? (H - h < HEADS ? H - h : HEADS) : HEADS);
+        }
+        if (live_tokens == 0) return;
+        if (RATIO == 128 && fused) {
+            // c8_attention's device plan: few live rows run as several
+            // partitions each (its rule, c8_attention.device_splits on the
+            // host, over this launch's work-groups), unless every row is a
+            // joint row.
+            int longest = 0;
+            for (int b0 = 0; b0 < live_batch; b0 += 64) {
+                const int b = b0 + (tid & 63) < live_batch ? b0 + (tid & 63) : live_batch - 1;
+                int len = cu[b + 1] >= 0 ? lens[b] : 0;
+#pragma unroll
+                for (int d = 1; d < 64; d *= 2) len = max(len, __shfl_xor(len, d));
+                longest = max(longest, uni(len));
+            }
+            const int live_rows = live_tokens * HG, tiles = 1 + (longest / RATIO + N - 1) / N;
+            if (tiles > 1 && PLAN_CUS / live_rows > 1 && !(resid && longest / RATIO <= N)) {
+                attention_item<RATIO, false, false, ANYH, false, true>(
+                    *reinterpret_cast<Shared *>(lds), cu_q, seq_lens, q_base, 0, batch_arg, 0, heads_arg, 1, rows_arg, grid,
+                    p, SharedKVDebug{0, 0, 0, 0, 0, 0, 0}, fused, rows_arg < grid ? rows_arg : grid);
+                return;
+            }
+        }
+        // The octets of the live rows are spread over the XCDs instead.
+        octets = (live_tokens * HG + CHUNK_ROWS - 1) / CHUNK_ROWS;
+        o = first_octet(x) + slot;
+        load_row();
+    }
+    // Octets that straddle requests.  A request that starts inside an octet
+    // is a tail: `tails` of them, `crowded` if some octet holds two.
+    // Work-groups that would have nothing to do in the last round of octets
+    // take the tails, one each, if they suffice or an octet is crowded (then
+    // further rounds take the rest).  Otherwise an octet takes its two
+    // requests at once (`pairs`, below).
+    auto is_tail = [&](int c0, int c1) {
+        return c0 >= 0 && c0 < live_tokens && c1 > c0 && c0 * HG % CHUNK_ROWS != 0;
+    };
+    int tails = 0;
+    bool crowded = false;
+    auto count_tails = [&](int c0, int c1, bool there) {
+        const bool mine = there && is_tail(c0, c1);
+        tails += __popcll(__ballot(mine));
+        crowded |= __ballot(mine && c1 < live_tokens && c1 * HG / CHUNK_ROWS == c0 * HG / CHUNK_ROWS) != 0;
+    };
+    count_tails(my_cu0, my_cu1, (tid & 63) < live_batch);
+    for (int b0 = 64; b0 < live_batch; b0 += 64) {
+        const int b = b0 + (tid & 63) < live_batch ? b0 + (tid & 63) : live_batch - 1;
+        count_tails(cu[b], cu[b + 1], b0 + (tid & 63) < live_batch);
+    }
+    int idle = 0, my_idle = -1;   // work-groups without an octet in their XCD's last round, and this one's number
+    for (int xcd = 0; xcd < 8; ++xcd) {
+        const int mine = first_octet(xcd + 1) - first_octet(xcd), used = mine % per_xcd;
+        if (mine && !used) continue;
+        if (xcd == x && slot >= used) my_idle = idle + slot - used;
+        idle += per_xcd - used;
+    }
+    const bool split = tails <= idle || crowded;
+    // Token at which tail `e` starts.
+    auto tail_start = [&](int e) {
+        int seen = 0;
+        for (int b0 = 0; b0 < live_batch; b0 += 64) {
+            const int b = b0 + (tid & 63) < live_batch ? b0 + (tid & 63) : live_batch - 1;
+            const int c0 = b0 ? cu[b] : my_cu0, c1 = b0 ? cu[b + 1] : my_cu1;
+            const uint64_t mask = __ballot(b0 + (tid & 63) < live_batch && is_tail(c0, c1));
+            const int n = __popcll(mask);
+            if (e < seen + n) {
+                const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+                const uint64_t at = __ballot((mask >> (tid & 63) & 1) && below == e - seen);
+                return __builtin_amdgcn_readlane(c0, __builtin_ctzll(at));
+            }
+            seen += n;
+        }
+        return -1;
+    };
+    const int past_octet = first_octet(x + 1);
+    int first = ANYH ? CHUNK_ROWS * o / HG : CHUNK_ROWS * o;
+    bool tail = false;
+    int next_tail = my_idle >= 0 ? my_idle : idle + (int)blockIdx.x;
+    // The work-group's next tail; false when there is none.
+    auto take_tail = [&]() {
+        if (!split || next_tail >= tails) return false;
+        first = tail_start(next_tail);
+        next_tail = next_tail < idle ? idle + (int)blockIdx.x : next_tail + (int)grid;
+        tail = true;
+        o = first * HG / CHUNK_ROWS;
+        load_row();
+        const int c1 = find_request(first).c1;
+        stop = c1 < stop ? c1 : stop;
+        return true;
+    };
+    if (o >= past_octet && !take_tail()) return;
+    *reinterpret_cast<f32x2 *>(&s.scale[tid >> 8][(tid & 255) * 2]) = scale_pair;
+
+    // The next octet or tail of the work-group, its rows' Q on its way; false
+    // when there is none.
+    auto next_item = [&]() {
+        if (tail || o + per_xcd >= past_octet) return take_tail();
+        o += per_xcd;
+        load_row();
+        first = ANYH ? CHUNK_ROWS * o / HG : CHUNK_ROWS * o;
+        return true;
+    };
+
+    for (bool more = true; more;) {
+        {
+            if (first >= stop || first >= live_tokens) {
+                more = next_item();
+                continue;
+            }
+            const int start = ANYH ? CHUNK_ROWS * o / HG : CHUNK_ROWS * o;   // the octet's first token
+            // Per-lane values derive from an opaque copy of the lane index, so
+            // that none is held in a register across the loop.
+            int lane = tid & 63;
+            asm volatile("" : "+v"(lane));
+            const int g = lane >> 4, n = lane & 15;
+            // Tokens of no live request and negative positions (reference.py:
+            // 104-105 rejects them) are zero.
+            const Request r0 = find_request(first);
+            if (r0.batch < 0 || r0.len - r0.c1 + first < 0) {
+                if (t == first) zero_row(t, hbase, hlive);
+                ++first;
+                continue;
+            }
+            // ---- the octet's lists (reference.py:228-253) ----
+            // Segment i: tokens [from[i], past[i]) of one request, their
+            // window rows lo0[i] .. (span[i] of them) and compressed rows.
+            int batch[2], back[2], from[2], past[2], lo0[2], span[2], all_rows[2], tiles[2];
+            auto segment = [&](int i, int token, const Request &r) {
+                batch[i] = r.batch;
+                back[i] = r.len - r.c1;                                      // position of token t: back + t
+                from[i] = token;
+                past[i] = r.c1 < stop ? r.c1 : stop;
+                past[i] = past[i] < live_tokens ? past[i] : live_tokens;
+                lo0[i] = back[i] + token + 1 > WINDOW ? back[i] + token + 1 - WINDOW : 0;
+                span[i] = back[i] + past[i] - lo0[i];
+                all_rows[i] = RATIO == 128 ? (back[i] + past[i]) / RATIO : 0;   // of its last token
+                tiles[i] = (all_rows[i] + N - 1) / N;
+            };
+            segment(0, first, r0);
+            if (split && !tail && first != start && first == r0.c0) {   // a tail, taken elsewhere
+                first = past[0];
+                continue;
+            }
+            batch[1] = back[1] = from[1] = past[1] = lo0[1] = span[1] = all_rows[1] = tiles[1] = 0;
+            // An octet that straddles two requests takes both windows at
+            // once, one in each buffer, unless there are joint rows (a joint
+            // row needs its window and its tile together).
+            bool two = false;
+            if (!split && past[0] < stop && past[0] < live_tokens) {
+                const Request r1 = find_request(past[0]);
+                if (r1.batch >= 0 && r1.len - r1.c1 + past[0] >= 0) {
+                    segment(1, past[0], r1);
+                    auto may_join = [&](int i) { return (back[i] + from[i] + 1) / RATIO <= N && all_rows[i] > 0; };
+                    two = RATIO == 1 || !resid || !(may_join(0) || may_join(1));
+                }
+            }
+            const int done = two ? past[1] : past[0];
+            const bool active = first <= t && t < done;
+            const int which = two && t >= past[0] ? 1 : 0;
+            const int position = active ? back[which] + t : 0;
+            const int own_first = position + 1 > WINDOW ? position + 1 - WINDOW : 0;
+            const int shift = active ? own_first - lo0[which] : 0;
+            const int own_window = position + 1 - own_first;
+            const int own_rows = RATIO == 128 && active ? (position + 1) / RATIO : 0;
+            // Table entries of the window's rows (row pair wave + 8 i: lanes
+            // 0-31 the first row, 32-63 the second) and of 64 compressed
+            // pages (16 tiles) are on their way during the first encode.
+            constexpr int PAIRS = (CHUNK_UNION / 2 + CHUNK_ROWS - 1) / CHUNK_ROWS;
+            int wpage[PAIRS];
+            auto read_window = [&](int sg) {
+                const __attribute__((address_space(1))) int32_t *otab =
+                    gptr<int32_t>(p.oriTable) + (int64_t)batch[sg] * p.oriTableWidth;
+#pragma unroll
+                for (int i = 0; i < PAIRS; ++i) {
+                    const int u = 2 * (wave + CHUNK_ROWS * i) + (lane >> 5), idx = lo0[sg] + u;
+                    wpage[i] = u < span[sg] && idx / BLOCK_ROWS < (int)p.oriTableWidth ? otab[idx / BLOCK_ROWS] : -1;
+                }
+            };
+            auto copy_window = [&](int sg) {
+#pragma unroll
+                for (int i = 0; i < PAIRS; ++i) {
+                    const int pair = wave + CHUNK_ROWS * i, u = 2 * pair + (lane >> 5), idx = lo0[sg] + u;
+                    if (2 * pair >= span[sg]) continue;
+                    const bool ok = (uint32_t)wpage[i] < p.oriPages;
+                    const uint64_t row_at =
+                        ok ? p.ori + (uint64_t)(uint32_t)wpage[i] * p.oriStride + (uint64_t)((idx % BLOCK_ROWS) * D) : p.q;
+                    dma16<false>(row_at + (uint64_t)(((lane & 31) ^ (u & 15)) << 4),
+                                 (uint32_t)uni((int)((uint32_t)(uintptr_t)buf + sg * CHUNK_UNION * D + 2 * pair * D)));
+                }
+                // Rows on no readable page, noted only when there are some.
+                bool bad = false;
+#pragma unroll
+                for (int i = 0; i < PAIRS; ++i)
+                    bad |= 2 * (wave + CHUNK_ROWS * i) + (lane >> 5) < span[sg] && (uint32_t)wpage[i] >= p.oriPages;
+                s.bad[sg][wave] = __ballot(bad) != 0;
+#pragma unroll
+                for (int i = 0; i < PAIRS; ++i)
+                    if ((lane & 31) == 0 && 2 * (wave + CHUNK_ROWS * i) < span[sg])
+                        s.window_ok[sg][2 * (wave + CHUNK_ROWS * i) + (lane >> 5)] = (uint32_t)wpage[i] < p.oriPages;
+            };
+            int entries = -1;
+            auto read_entries = [&](int sg, int k) {   // pages 4 k .. 4 k + 63 of segment sg
+                const int e = 4 * k + lane;
+                entries = e < (int)p.cmpTableWidth && e * BLOCK_ROWS < all_rows[sg]
+                              ? gptr<int32_t>(p.cmpTable)[(int64_t)batch[sg] * p.cmpTableWidth + e]
+                              : -1;
+            };
+            // Copies of compressed tile k of segment sg to buffer b: wave w
+            // moves rows 16 w .. 16 w + 15, half of page 4 k + w / 2.  Rows
+            // past the list or on no page are left as they are (masked
+            // later).  Returns which of the tile's four pages are there.
+            auto copy_tile = [&](int sg, int k, int b) {
+                if (!(k & 15) && (sg || k)) read_entries(sg, k);
+                const int page = __builtin_amdgcn_readlane(entries, 4 * (k & 15) + (wave >> 1));
+                const uint32_t there = (uint32_t)(__ballot(entries >= 0) >> (4 * (k & 15))) & 15u;
+                if (page < 0 || N * k + 16 * wave >= all_rows[sg]) return there;
+                const uint64_t base = p.cmp + (uint64_t)page * p.cmpStride + (uint64_t)((wave & 1) * 16 * D);
+                const uint32_t dst = (uint32_t)(uintptr_t)buf + b * CHUNK_UNION * D + 16 * wave * D;
+#pragma unroll
+                for (int r = 0; r < 8; ++r)
+                    dma16_at(base, (uint32_t)((2 * r + (lane >> 5)) * D + (((lane & 31) ^ (2 * r + (lane >> 5))) << 4)),
+                             (uint32_t)uni((int)(dst + 2 * r * D)));
+                return there;
+            };
+
+            // Row state (heads 2g and 2g + 1, columns 16 j + n): maximum,
+            // denominator, numerator.
+            float mx[2], den[2], num[2][32] = {};
+            v4i qa0[8] = {}, qa1[8] = {};
+            float asc0[2] = {}, asc1[2] = {};
+
+            // P codes of a tile (reference.py:304-312) from its weights: 16 bytes
+            // per key, this lane writing MFMA rows 4g .. 4g + 3.
+            auto put_codes = [&](const float (&w)[8][2]) {
+#pragma unroll
+                for (int b = 0; b < 8; ++b) {
+                    float hi[2], lo[2];
+#pragma unroll
+                    for (int hh = 0; hh < 2; ++hh) {
+                        const float x = w[b][hh] * 127.0f;
+                        hi[hh] = x + MAGIC;
+                        lo[hh] = resid ? (x - (hi[hh] - MAGIC)) * 127.0f + MAGIC : 0.0f;
+                    }
+                    *(lds_u32 *)(pw + (16 * b + n) * 16 + 4 * g) = low_bytes(hi[0], lo[0], hi[1], lo[1]);
+                }
+                asm volatile("" ::: "memory");
+            };
+            // P codes in the MFMA A layout.  Keys of a 64-key block: lane group g
+            // takes keys 8g .. 8g + 7 and 32 + 8g .. 32 + 8g + 7 (any assignment of
+            // keys gives the same integers, as long as V uses the same).
+            auto get_codes = [&](v4i (&pa)[2]) {
+                const lds_i8 *at = pw + (8 * g + (n >> 1)) * 16 + 8 * (n & 1);
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) {
+                    const v2i a = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(at + kb * 1024));
+                    const v2i b = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(at + kb * 1024 + 512));
+                    pa[kb] = v4i{a.x, a.y, b.x, b.y};
+                }
+                asm volatile("" ::: "memory");
+            };
+            // S = Q K^T of the row's 128 keys, tile rows shift .. shift + 127, as
+            // logits (reference.py:286-303); key 16 b + n counts when below `live`
+            // and its row is readable (32-key pages `pages`, or the window's rows).
+            auto logits = [&](const lds_i8 *tb, int shift, int live, uint32_t pages, bool in_window, const v4i (&qa)[8],
+                          const float (&asc)[2], float (&lg)[8][2]) {
+                int lx = lane;
+                asm volatile("" : "+v"(lx));
+                const int gx = lx >> 4, nx = lx & 15;
+                const int r0 = shift + nx, f = r0 & 15;
+                const lds_i8 *at = tb + r0 * D;
+                uint32_t off[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) off[j] = (uint32_t)((4 * j + gx) ^ f) << 4;
+                // Step st: key blocks 2 (st / 2) and + 1, channels 256 (st % 2)
+                // and up; the next step's reads are in flight during its MFMAs.
+                v4i k[2][8], acc[2];
+                auto fetch = [&](int st) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+                            k[st & 1][2 * j + i] =
+                                *(const lds_v4i *)(at + off[4 * (st & 1) + j] + (2 * (st >> 1) + i) * 16 * D);
+                };
+                fetch(0);
+#pragma unroll
+                for (int st = 0; st < 8; ++st) {
+                    if (st + 1 < 8) fetch(st + 1);
+                    if (!(st & 1)) acc[0] = acc[1] = v4i{0, 0, 0, 0};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+                            acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa[4 * (st & 1) + j], k[st & 1][2 * j + i], acc[i], 0, 0, 0);
+                    if (st & 1) {
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            const int b = st - 1 + i;
+                            const int most = (pages >> (b >> 1)) & 1u ? live : 0;
+                            const bool valid = nx < most - 16 * b;
+#pragma unroll
+                            for (int hh = 0; hh < 2; ++hh) {
+                                float dots = (float)acc[i][2 * hh];
+                                dots = dots + (float)acc[i][2 * hh + 1] * (float)(1.0 / 127.0);
+                                float l = dots * asc[hh];
+                                asm volatile("" : "+v"(l));   // a select, not a branch
+                                lg[b][hh] = valid ? l : -1e30f;
+                            }
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (in_window && __ballot(s.bad[which][lane & (CHUNK_ROWS - 1)])) {
+#pragma unroll
+                    for (int b = 0; b < 8; ++b)
+                        if (16 * b + n < live && !s.window_ok[which][shift + 16 * b + n]) lg[b][0] = lg[b][1] = -1e30f;
+                }
+            };
+            auto row_max = [&](const float (&lg)[8][2], int hh) {
+                float m = lg[0][hh];
+#pragma unroll
+                for (int b = 1; b < 8; ++b) m = fmaxf(m, lg[b][hh]);
+                return m;
+            };
+            // Pairwise weight sum over the tile's 128 positions.
+            auto tree = [&](const float (&w)[8][2], int hh) {
+                float t[8];
+#pragma unroll
+                for (int b = 0; b < 8; ++b) t[b] = row16_tree_sum(w[b][hh]);
+                return ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+            };
+            auto sink_factor = [&](const float (&mnew)[2], float (&factor)[2]) {
+                const bool odd = n & 1;   // exp(max_old - max_new), one exponential per lane pair
+                const float mine = sk_expf_nonpos(odd ? mx[1] - mnew[1] : mx[0] - mnew[0]);
+                const float other = dpp<DPP_XOR1>(mine);
+                factor[0] = odd ? other : mine;
+                factor[1] = odd ? mine : other;
+            };
+            // P V over the tile, 64 columns at a time, each followed by its FP32
+            // epilogue: done(hh, column block, V_hi, V_lo, channel scale).
+            auto pv = [&](const lds_i8 *tb, int shift, int kind, auto done) {
+                v4i pa[2];
+                get_codes(pa);
+                int lx = lane;
+                asm volatile("" : "+v"(lx));
+                const int gx = lx >> 4, nx = lx & 15;
+                const int r0 = shift + 8 * gx + (nx >> 1), f = r0 & 15;
+                const lds_i8 *at = tb + r0 * D + 8 * (nx & 1);
+                const float *sc = s.scale[kind] + nx;
+constexpr int PC = 2;
+                // Column chunk jc (16 PC columns): the next chunk's reads are in flight
+                // during its MFMAs and epilogue.
+                v2i bb[2][4 * PC];
+                auto fetch = [&](int jc) {
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int j = 0; j < PC; ++j) {
+                            const int c = PC * jc + j;
+                            const lds_i8 *cat = at + (((c & 15) ^ f) << 4);
+                            bb[jc & 1][PC * kb + j] =
+                                __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(cat + (c & 16) * 16 + kb * 64 * D));
+                            bb[jc & 1][2 * PC + PC * kb + j] =
+                                __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(cat + (c & 16) * 16 + kb * 64 * D + 32 * D));
+                        }
+                };
+                fetch(0);
+#pragma unroll
+                for (int jc = 0; jc < 32 / PC; ++jc) {
+                    if (jc + 1 < 32 / PC) fetch(jc + 1);
+                    v4i acc[PC];
+#pragma unroll
+                    for (int j = 0; j < PC; ++j) acc[j] = v4i{0, 0, 0, 0};
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int j = 0; j < PC; ++j) {
+                            const v2i lo8 = bb[jc & 1][PC * kb + j], hi8 = bb[jc & 1][2 * PC + PC * kb + j];
+                            acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(pa[kb], v4i{lo8.x, lo8.y, hi8.x, hi8.y}, acc[j], 0, 0, 0);
+                        }
+#pragma unroll
+                    for (int j = 0; j < PC; ++j) {
+                        const float scale = sc[16 * (PC * jc + j)];
+#pragma unroll
+                        for (int hh = 0; hh < 2; ++hh) done(hh, PC * jc + j, acc[j][2 * hh], acc[j][2 * hh + 1], scale);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            // One tile of the online softmax (reference.py:280-316).
+            auto run_tile = [&](const lds_i8 *tb, int shift, int live, uint32_t pages, auto kind_c, const v4i (&qa)[8],
+                                const float (&asc)[2]) {
+                constexpr int kind = decltype(kind_c)::value;
+                float lg[8][2], mnew[2], factor[2];
+                logits(tb, shift, live, pages, kind == 0, qa, asc, lg);
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh)
+                    mnew[hh] = fkey_value(max(fkey(mx[hh]), row16_max_key(fkey(row_max(lg, hh)))));
+                sink_factor(mnew, factor);
+#pragma unroll
+                for (int b = 0; b < 8; ++b)
+#pragma unroll
+                    for (int hh = 0; hh < 2; ++hh) lg[b][hh] = sk_expf_nonpos(lg[b][hh] - mnew[hh]);
+                put_codes(lg);
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    den[hh] = den[hh] * factor[hh] + tree(lg, hh);
+                    mx[hh] = mnew[hh];
+                }
+                pv(tb, shift, kind, [&](int hh, int c, int hi, int lo, float scale) {
+                    float dots = (float)hi;
+                    dots = dots + (float)lo * (float)(1.0 / 127.0);
+                    num[hh][c] = (kind ? num[hh][c] : 0.0f) * factor[hh] + dots * scale * (float)(1.0 / 127.0);
+                });
+            };
+            // Joint row (reference.py:254-267, joint_quantized_row 175-207): one
+            // softmax over the window's keys and the one compressed tile's.
+            auto run_joint = [&](int shift, int live0, int live1, uint32_t pages) {
+                float l0[8][2], l1[8][2], mnew[2], factor[2];
+                logits(buf, shift, live0, 15u, true, qa0, asc0, l0);
+                logits(buf + CHUNK_UNION * D, 0, live1, pages, false, qa1, asc1, l1);
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh)
+                    mnew[hh] = fkey_value(max(fkey(mx[hh]), row16_max_key(fkey(fmaxf(row_max(l0, hh), row_max(l1, hh))))));
+                sink_factor(mnew, factor);
+#pragma unroll
+                for (int b = 0; b < 8; ++b)
+#pragma unroll
+                    for (int hh = 0; hh < 2; ++hh) {
+                        l0[b][hh] = sk_expf_nonpos(l0[b][hh] - mnew[hh]);
+                        l1[b][hh] = sk_expf_nonpos(l1[b][hh] - mnew[hh]);
+                    }
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    den[hh] = factor[hh] + (tree(l0, hh) + tree(l1, hh));
+                    mx[hh] = mnew[hh];
+                }
+                put_codes(l0);
+                pv(buf, shift, 0, [&](int hh, int c, int hi, int lo, float scale) {
+                    float dots = (float)hi;
+                    dots = dots + (float)lo * (float)(1.0 / 127.0);
+                    num[hh][c] = 0.0f + dots * (scale * (float)(1.0 / 127.0));   // the output starts at 0
+                });
+                put_codes(l1);
+                pv(buf + CHUNK_UNION * D, 0, 1, [&](int hh, int c, int hi, int lo, float scale) {
+                    float dots = (float)hi;
+                    dots = dots + (float)lo * (float)(1.0 / 127.0);
+                    num[hh][c] = num[hh][c] + dots * (scale * (float)(1.0 / 127.0));
+                });
+            };
+            // ---- Q folding and residual split per kind (reference.py:274-279) ----
+            const bool odd = n & 1;
+            auto encode = [&](int kind, v4i (&qa)[8], float (&asc)[2]) {
+                const float *scale = s.scale[kind] + 16 * g + 8 * (n & 1);
+                float f[8][8], amax = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t w[4] = {(uint32_t)qraw[j].x, (uint32_t)qraw[j].y, (uint32_t)qraw[j].z, (uint32_t)qraw[j].w};
+                    const f32x4 s0 = *reinterpret_cast<const f32x4 *>(scale + 64 * j);
+                    const f32x4 s1 = *reinterpret_cast<const f32x4 *>(scale + 64 * j + 4);
+                    const float sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        f[j][e] = __uint_as_float(e & 1 ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16) * sc[e];
+                        amax = fmaxf(amax, fabsf(f[j][e]));
+                    }
+                }
+                amax = fmaxf(amax, dpp<DPP_XOR1>(amax));
+                amax = fmaxf(amax, __shfl_xor(amax, 16));
+                amax = fmaxf(amax, __shfl_xor(amax, 32));
+                float alpha = amax * (float)(1.0 / 127.0);
+                alpha = alpha < 1e-12f ? 1e-12f : alpha;
+                const float inv = 1.0f / alpha;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    float hi[8], lo[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float v = clamp127(f[j][e] * inv);
+                        hi[e] = v + MAGIC;
+                        lo[e] = resid ? (v - (hi[e] - MAGIC)) * 127.0f + MAGIC : 0.0f;
+                    }
+                    const int h0 = (int)low_bytes(hi[0], hi[1], hi[2], hi[3]), h1 = (int)low_bytes(hi[4], hi[5], hi[6], hi[7]);
+                    const int l0 = (int)low_bytes(lo[0], lo[1], lo[2], lo[3]), l1 = (int)low_bytes(lo[4], lo[5], lo[6], lo[7]);
+                    const int l0x = dpp_i<DPP_XOR1>(l0), l1x = dpp_i<DPP_XOR1>(l1);
+                    const int h0x = dpp_i<DPP_XOR1>(h0), h1x = dpp_i<DPP_XOR1>(h1);
+                    qa[j] = v4i{odd ? l0x : h0, odd ? l1x : h1, odd ? l0 : h0x, odd ? l1 : h1x};
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                asc[0] = __shfl(alpha, 4 * g) * p.softmaxScale;
+                asc[1] = __shfl(alpha, 4 * g + 2) * p.softmaxScale;
+            };
+            read_window(0);
+            if (RATIO == 128) read_entries(0, 0);
+            lds_barrier();   // the scales are there; every wave is done with the buffers
+            if (active) {
+                encode(0, qa0, asc0);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(qa0[j]));   // encoded here, not after the waits
+            }
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // the table entries (vmcnt 0), before the copies below
+            copy_window(0);
+            if (two) {
+                read_window(1);
+                __builtin_amdgcn_s_waitcnt(0x0F70);
+                copy_window(1);
+            }
+            uint32_t pages = 0;
+            if (RATIO == 128 && !two && tiles[0]) pages = copy_tile(0, 0, 1);
+            if (RATIO == 128 && active) {
+                encode(1, qa1, asc1);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(qa1[j]));
+            }
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                mx[hh] = sink[hh];
+                den[hh] = 1.0f;
+            }
+            vm_wait<0>();
+            lds_barrier();   // windows and tile 0 have landed for every wave
+            const bool joint = RATIO == 128 && resid && own_rows >= 1 && own_rows <= N;
+            if (active) {
+                if (joint)
+                    run_joint(shift, own_window, own_rows, pages);
+                else
+                    run_tile(buf + which * CHUNK_UNION * D, shift, own_window, 15u, std::integral_constant<int, 0>{}, qa0, asc0);
+            }
+            if (RATIO == 128) {
+                int sg = two && !tiles[0] ? 1 : 0, k = 0;
+                if (two && tiles[sg]) {
+                    lds_barrier();   // every wave is done with the windows
+                    pages = copy_tile(sg, 0, 1);
+                }
+                // Tiles in turn, tile `it` of them in buffer (it + 1) % 2,
+                // the next one on its way during it.
+#pragma nounroll
+                for (int it = 0; k < tiles[sg]; ++it) {
+                    vm_wait<0>();
+                    lds_barrier();   // the tile has landed; every wave is done with the other buffer
+                    const int at_sg = sg, at_k = k;
+                    const uint32_t at_pages = pages;
+                    if (++k >= tiles[sg] && two && sg == 0 && tiles[1]) { sg = 1; k = 0; }
+                    if (k < tiles[sg]) pages = copy_tile(sg, k, it & 1);
+                    const int live = own_rows - N * at_k < N ? own_rows - N * at_k : N;
+                    if (active && which == at_sg && !joint && live > 0)
+                        run_tile(buf + ((it + 1) & 1) * CHUNK_UNION * D, 0, live, at_pages, std::integral_constant<int, 1>{},
+                                 qa1, asc1);
+                }
+            }
+            // The next rows' Q is on its way during the output.
+            const int out_t = t, out_hbase = hbase, out_hlive = hlive;
+            first = done;
+            if (first >= stop || first >= live_tokens) more = next_item();
+            else load_row();
+            // ---- finalize (reference.py:317-323 with one partition) ----
+            lds_barrier();   // the buffers are free
+            if (active) {
+                int8_t *stage = s.buf[0] + wave * HEADS * OUT_STRIDE;
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    // Columns 16 c + n and 16 (c + 1) + n: lanes n and n ^ 1
+                    // exchange one of them, so that each writes two neighbours
+                    // (even lanes of block c, odd lanes of block c + 1).
+                    const float r = 1.0f / den[hh];
+                    const uint32_t pick = n & 1 ? 0x03020706u : 0x05040100u;
+                    uint32_t *to = reinterpret_cast<uint32_t *>(stage + (2 * g + hh) * OUT_STRIDE) + 8 * (n & 1) + (n >> 1);
+#pragma unroll
+                    for (int c = 0; c < 32; c += 2) {
+                        const uint32_t mine = pack_bf16(div_by(num[hh][c], den[hh], r), div_by(num[hh][c + 1], den[hh], r));
+                        const uint32_t other = (uint32_t)dpp_i<DPP_XOR1>((int)mine);
+                        to[8 * c] = __builtin_amdgcn_perm(other, mine, pick);
+                    }
+                    if (p.lse && n == 0 && 2 * g + hh < out_hlive)
+                        reinterpret_cast<float *>(p.lse)[(int64_t)out_t * H + out_hbase + 2 * g + hh] = mx[hh] + logf(den[hh]);
+                }
+                asm volatile("" ::: "memory");
+                v4i *o = reinterpret_cast<v4i *>(reinterpret_cast<uint16_t *>(p.out) + ((int64_t)out_t * H + out_hbase) * D);
+#pragma unroll
+                for (int h = 0; h < HEADS; ++h)
+                    if (!ANYH || h < out_hlive)
+                        __builtin_nontemporal_store(*reinterpret_cast<const v4i *>(stage + h * OUT_STRIDE + 16 * lane), o + 64 * h + lane);
+            }
+        }
+    }
+}
+
 // ---- INT8 cache writer (cache_write.cpp:9-88): one wave per update row ----
 template <typename Index, bool Paired>
 __global__ void __launch_bounds__(256)
@@ -2900,6 +3693,16 @@ bool xcd_local_dispatch(hipStream_t stream, bool may_probe)
     return ok;
 }
 
+// Launches of c8_chunk: a work-group takes eight rows in about the time of one
+// (window-only 15 us, C128 at 8 K / 32 K context 24 / 30 us for any row count
+// up to 2048), so they need enough rows.  Window-only: 1024 rows take 16.1 us
+// on c8_chunk and 14.4 on c8_rows, 1500 rows 16.5 and 20.2.  C128: 700 rows
+// 24.6 and 24.3 at 8 K (30.8 and 30.7 at 32 K) against c8_attention, 1024 rows
+// 24.8 and 31.9 (30.8 and 40.6).  And the rows of a work-group have to come
+// from few requests (1024 rows of 128 requests are no slower, 512 rows of
+// them are), which the launch only knows on average.
+constexpr uint32_t CHUNK_MIN_WINDOW = 1024, CHUNK_MIN_C128 = 768, CHUNK_REQUEST_TOKENS = 16;
+
 template <bool DEBUG, bool ANYH>
 void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDebug &dbg, bool slots, uint32_t grid,
                     uint32_t splits, uint32_t rows, uint32_t fused, bool small_entry)
@@ -2917,13 +3720,21 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
     // they cost tiled C4 launches about 1 %.
     const bool joint4 = !DEBUG && !slots && a->heads <= HEADS &&
                         (small_entry || (uint64_t)a->cmpTableWidth * BLOCK_ROWS <= (uint64_t)N);
+    // Prefill-shaped C128 and window-only launches share KV tiles between
+    // neighbouring rows.
+    if (!DEBUG && !slots && splits == 1 && a->ratio != 4 &&
+        rows > (a->ratio == 1 ? CHUNK_MIN_WINDOW : CHUNK_MIN_C128) &&
+        (uint64_t)a->tokens >= (uint64_t)CHUNK_REQUEST_TOKENS * a->batch) {
+        const uint32_t cus = (uint32_t)PLAN_CUS;
+        hipLaunchKernelGGL((a->ratio == 1 ? &c8_chunk<1, ANYH> : &c8_chunk<128, ANYH>), dim3(cus), dim3(THREADS), 0, stream,
+                           a->cuQ, a->seqLens, a->q, a->batch, rows, cus, a->heads, *a, fused);
+        return;
+    }
     // One-partition C4 and window-only launches of more rows than CUs
     // (prefill, large decode batches) without explicit slots run two
-    // four-wave work-groups per CU taking rows in turn (c8_rows).  C128
-    // launches keep one work-group per row: their rows are three or fewer
-    // tiles in a prefill chunk, or joint rows, and c8_attention's two-tile
-    // ring measured faster on them (C128 prefill chunk 80 against 85 us,
-    // joint rows 63 against 110, decode of 512 rows 51 against 72).
+    // four-wave work-groups per CU taking rows in turn (c8_rows).  Other C128
+    // launches keep one work-group per row: c8_attention's two-tile ring
+    // measured faster on them (decode of 512 rows 51 against 72 us).
     const bool persist = !DEBUG && !slots && splits == 1 && rows > (uint32_t)PLAN_CUS &&
                          (a->ratio == 1 || (a->ratio == 4 && !joint4));
     if (persist) {

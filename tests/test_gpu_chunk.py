@@ -1,0 +1,91 @@
+"""Prefill-shaped C128 and window-only launches (c8_chunk: one query row per
+wave, eight neighbouring rows of a work-group sharing their KV tiles): how the
+octets of rows meet requests, padding, joint rows, head groups and unreadable
+pages.  Bit-exact with the checker on the launch's plan; every launch here is
+large enough for that kernel (more than 1024 window-only rows or 768 C128 rows,
+16 query tokens per request on average)."""
+import sys
+
+import numpy as np
+import pytest
+
+from tests import workloads
+from tests.device_cases import joint_flags, query_subcase, run_hip, run_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, file=sys.stderr, flush=True)
+
+
+def padded(case, pad):
+    """The case at a graph's capacity: `pad` NaN query rows of an empty request."""
+    live = int(case["cu_q"][-1])
+    nan = np.full((pad,) + case["q"].shape[1:], 0x7FC0, np.uint16)
+    out = dict(case, q=np.concatenate([case["q"], nan]),
+               cu_q=np.concatenate([case["cu_q"], [live + pad]]).astype(np.int32),
+               seq_lens=np.concatenate([case["seq_lens"], [0]]).astype(np.int32))
+    for name in ("ori", "cmp"):
+        if out[name] is not None:
+            out[name].table = np.concatenate([out[name].table, out[name].table[:1]])
+    return out
+
+
+CASES = [
+    # name, ratio, queries, lengths, heads, padding rows
+    ("one_request", 1, [1041], [1041], 8, 0),                    # positions from 0 on, a last octet of one row
+    ("pairs", 1, [1041, 1007], [1500, 1030], 8, 0),              # 256 octets, one of two requests
+    ("pairs_c128", 128, [1041, 1007], [17600, 18000], 8, 0),     # the same, tiles of both in turn
+    ("joint_straddle", 128, [1041, 1007], [3000, 9000], 8, 0),   # joint rows: one request after the other
+    ("joint_edges", 128, [800], [16900], 8, 0),                  # rows of 127 to 132 compressed rows
+    ("tails", 128, [403, 5, 399], [20000, 300, 17000], 8, 3),    # requests that start inside octets
+    ("crowded", 1, [1020, 1, 1, 2, 1, 1023], [1100, 9, 700, 2, 131, 1200], 8, 0),   # several in one octet
+    ("many_requests", 1, [17] * 70, list(range(17, 17 + 70 * 9, 9)), 8, 5),         # more than one wave's metadata
+    ("keyless", 1, [700, 4, 400], [698, 1, 800], 8, 0),          # negative positions
+    ("head_groups", 128, [300, 101], [17000, 2500], 20, 2),      # three groups of eight, the last of four
+    ("four_heads", 1, [600, 500], [700, 2000], 4, 1),
+    ("replanned", 128, [30, 9], [20000, 700], 8, 900),           # few live rows: several partitions each
+    ("padded_joint", 128, [60, 9], [3000, 700], 8, 900),
+]
+
+
+@pytest.mark.parametrize("name,ratio,queries,lengths,heads,pad", CASES, ids=[c[0] for c in CASES])
+def test_chunk_launch_matches_checker(name, ratio, queries, lengths, heads, pad):
+    from npu_sparse_attn_sharedkv_int8 import c8_attention
+    say(f"[chunk] {name}")
+    case = workloads.make_case(90, ratio, queries, lengths, heads=heads)
+    launch = padded(case, pad) if pad else case
+    rows = launch["q"].shape[0] * ((heads + 7) // 8)
+    assert rows > (1024 if ratio == 1 else 768) and launch["q"].shape[0] >= 16 * len(launch["seq_lens"])
+    out, lse, op = run_hip(launch, splits=1)
+    plan, joint = op.device_splits(), joint_flags(launch, 1)
+    assert (plan > 1) == (name == "replanned")
+    live = int(case["cu_q"][-1])
+    assert not out[live:].any() and not lse[live:].any(), "padding rows are not zero"
+    dead = c8_attention.keyless_tokens(case["cu_q"], case["seq_lens"], live)
+    keep = [t for t in range(live) if not dead[t]]
+    assert not out[[t for t in range(live) if dead[t]]].any(), "keyless rows are not zero"
+    # The launch's own requests where the checker takes them, else one request per row.
+    sub = case if len(keep) == live else query_subcase(case, keep)
+    ref, ref_lse, _ = run_oracle(sub, plan, joint=joint)
+    diff = out[keep] != ref
+    assert not diff.any(), f"{int(diff.sum())} BF16 mismatches, rows {sorted(set(np.argwhere(diff)[:, 0]))[:8]}"
+    np.testing.assert_allclose(lse[keep], ref_lse, rtol=0, atol=2e-6)
+
+
+@pytest.mark.parametrize("ratio", [1, 128])
+def test_unreadable_pages_equal_the_general_path(ratio):
+    """Block-table entries past the pool (window) and negative ones
+    (compressed): the rows on them are masked, as in a launch of a few of the
+    same rows (c8_attention)."""
+    case = workloads.make_case(91, ratio, [1100], [18400 if ratio == 128 else 1300])
+    table = case["ori"].table
+    table[0, [table.shape[1] - 2, table.shape[1] - 9]] = case["ori"].pages + 3
+    if ratio == 128:
+        case["cmp"].table[0, [1, 4]] = -1
+    say(f"[chunk] unreadable pages, ratio {ratio}")
+    out, lse, op = run_hip(case, splits=1)
+    rows = list(range(3, 1100, 13)) + list(range(1092, 1100))
+    ref, ref_lse, few = run_hip(query_subcase(case, rows), splits=1)
+    assert (out[rows] == ref).all() and (lse[rows] == ref_lse).all()
