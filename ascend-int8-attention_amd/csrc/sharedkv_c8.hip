@@ -122,10 +122,11 @@ __device__ __forceinline__ float sk_expf_nonpos(float x)
 {
     // Evaluated without a branch: the series runs on a clamped argument and
     // the result is selected, which keeps both exponentials of a lane in one
-    // instruction stream.
-    const bool in_range = x >= -87.0f;
-    const float xr = in_range ? x : -87.0f;
-    float n = __builtin_rintf(xr * 1.44269504088896341f);
+    // instruction stream.  NaN is not below -87 and runs through the series
+    // (v_cvt_i32_f32 turns it into 0).
+    const bool below = x < -87.0f;
+    const float xr = below ? -87.0f : x;
+    const float n = __builtin_rintf(xr * 1.44269504088896341f);
     float r = __builtin_fmaf(-n, 0.693145751953125f, xr);
     r = __builtin_fmaf(-n, 1.42860682030941723212e-6f, r);
     float p = 1.0f / 40320.0f;
@@ -137,11 +138,13 @@ __device__ __forceinline__ float sk_expf_nonpos(float x)
     p = __builtin_fmaf(p, r, 0.5f);
     p = __builtin_fmaf(p, r, 1.0f);
     p = __builtin_fmaf(p, r, 1.0f);
-    float e = __builtin_ldexpf(p, (int)n);
+    int exponent;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(exponent) : "v"(n));
+    float e = __builtin_ldexpf(p, exponent);
     // Keeps the series unconditional: without it the compiler turns the
     // select below back into a branch around the series.
     asm volatile("" : "+v"(e));
-    return in_range ? e : (x != x ? x : 0.0f);
+    return below ? 0.0f : e;
 }
 
 __device__ __forceinline__ float clamp127(float x) { return fminf(fmaxf(x, -127.0f), 127.0f); }
@@ -1512,11 +1515,130 @@ c8_merge(const SharedKVArgs p, uint32_t splits)
                 H - hbase < HEADS ? H - hbase : HEADS);
 }
 
+typedef __attribute__((address_space(3))) v4i lds_v4i;
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+// x rounded to the nearest even integer sits in the low bits of x + MAGIC
+// (|x| < 2^22), so the low byte of the sum is the INT8 code.
+constexpr float MAGIC = 12582912.0f;
+__device__ __forceinline__ uint32_t low_bytes(float a, float b, float c, float d)
+{
+    const uint32_t ab = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x0c0c0400u);
+    const uint32_t cd = __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(c), 0x04000c0cu);
+    return ab | cd;
+}
+
+// num / den, correctly rounded, from the correctly rounded reciprocal r of
+// den: the FMA residual of the product corrects it (Markstein, 1990; den is
+// a softmax denominator, so no operand is subnormal).
+__device__ __forceinline__ float div_by(float num, float den, float r)
+{
+    const float q = num * r;
+    // An infinite quotient's residual is NaN; the median turns that into a
+    // finite number, which leaves the infinity as it is.
+    const float e = __builtin_amdgcn_fmed3f(__builtin_fmaf(-q, den, num), -3.0e38f, 3.0e38f);
+    return __builtin_fmaf(e, r, q);
+}
+
+// ---- launch metadata by wave ballots ----
+// Every wave holds the first 64 requests' (cu[b], cu[b + 1], len[b]) in lane
+// b; later requests are read in groups of 64.  No barrier, no LDS.
+typedef const __attribute__((address_space(1))) int32_t *global_i32;
+struct LiveShape {
+    int batch, end;   // requests up to the last with seq_len > 0 and cu_q >= 0, and its cu_q end (0: none)
+};
+__device__ __forceinline__ LiveShape live_shape(global_i32 cu, global_i32 lens, int batch_n, int my_cu1, int my_len)
+{
+    const int lane = threadIdx.x & 63;
+    LiveShape live{0, 0};
+    const uint64_t there = __ballot(lane < batch_n && my_len > 0 && my_cu1 >= 0);
+    if (there) {
+        live.batch = 64 - __builtin_clzll(there);
+        live.end = __builtin_amdgcn_readlane(my_cu1, live.batch - 1);
+    }
+    for (int b0 = 64; b0 < batch_n; b0 += 64) {
+        const int b = b0 + lane < batch_n ? b0 + lane : batch_n - 1;
+        const int c1 = cu[b + 1];
+        const uint64_t more = __ballot(b0 + lane < batch_n && lens[b] > 0 && c1 >= 0);
+        if (more) {
+            live.batch = b0 + 64 - __builtin_clzll(more);
+            live.end = __builtin_amdgcn_readlane(c1, 63 - __builtin_clzll(more));
+        }
+    }
+    return live;
+}
+// The longest live sequence (of the requests live_shape counts).
+__device__ __forceinline__ int longest_live(global_i32 cu, global_i32 lens, int live_batch)
+{
+    const int lane = threadIdx.x & 63;
+    int longest = 0;
+    for (int b0 = 0; b0 < live_batch; b0 += 64) {
+        const int b = b0 + lane < live_batch ? b0 + lane : live_batch - 1;
+        int len = cu[b + 1] >= 0 ? lens[b] : 0;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) len = max(len, __shfl_xor(len, d));
+        longest = max(longest, uni(len));
+    }
+    return longest;
+}
+// The live request holding `token`.
+struct Request {
+    int batch, c0, c1, len;   // batch < 0: none
+};
+__device__ __forceinline__ Request find_request(global_i32 cu, global_i32 lens, int live_batch, int my_cu0, int my_cu1,
+                                                int my_len, int token)
+{
+    const int lane = threadIdx.x & 63;
+    const uint64_t hit = __ballot(lane < live_batch && my_cu0 <= token && token < my_cu1);
+    if (hit) {
+        const int b = __builtin_ctzll(hit);
+        return Request{b, __builtin_amdgcn_readlane(my_cu0, b), __builtin_amdgcn_readlane(my_cu1, b),
+                       __builtin_amdgcn_readlane(my_len, b)};
+    }
+    for (int b0 = 64; b0 < live_batch; b0 += 64) {
+        const int b = b0 + lane < live_batch ? b0 + lane : live_batch - 1;
+        const int c0 = cu[b], c1 = cu[b + 1], len = lens[b];
+        const uint64_t more = __ballot(b0 + lane < live_batch && c0 <= token && token < c1);
+        if (more) {
+            const int at = __builtin_ctzll(more);
+            return Request{b0 + at, __builtin_amdgcn_readlane(c0, at), __builtin_amdgcn_readlane(c1, at),
+                           __builtin_amdgcn_readlane(len, at)};
+        }
+    }
+    return Request{-1, 0, 0, 0};
+}
+
 // ---- c8_rows: one-partition launches of many query rows ----
 // The same numerics as c8_attention with one partition (128-key tiles,
 // reference.py:210-323), laid out so that two work-groups share a CU: four
 // waves and one tile buffer each (80 KiB of LDS), each work-group taking rows
 // r, r + grid, ... in turn.
+// A row's tiles are a chain (QK -> tile maximum -> exponentials and P codes
+// -> PV) through work-group barriers; with two rows per CU the other
+// work-group computes while this one waits.  The next tile's rows are on
+// their way to registers (whole rows, 64 VGPRs a lane) during the chain and
+// written to the tile buffer when it is free, so that a tile never waits for
+// memory.  Each wave takes 32 keys in QK (the rows it copied: no barrier
+// before it) and 128 output columns in PV.
+// Bound by instruction issue: 391 VALU instructions a wave and tile (most of
+// them the FP32 sequence), VALU 62 % and LDS 40 % busy; with every row an L2
+// hit a prefill chunk takes the same time.  Eight waves a work-group at 128
+// VGPRs were slower (130 against 116 us on the chunk below).
+// Measured on MI355X, LDS DMA copies and rows of eight heads -> this: decode
+// of 512 C4 rows 55 -> 52 us, 1024 rows 85.5 -> 77.4; 512 and 1024 window-only
+// rows 8.6 -> 7.9 and 14.5 -> 12.9; C4 prefill chunk B = 1 x T = 2048 117 ->
+// 116; of 16 heads, T = 1024 118 -> 75; decode of 256 sequences of 32 heads
+// 78 -> 48.
+// Rows lie in LDS as in c8_chunk (row u at u * 512, 16-byte chunks swizzled
+// by u & 15), P codes key-major.
+// WIDE: more than eight heads.  There are no residual codes then
+// (reference.py:221-222), so the sixteen MFMA rows hold sixteen heads' codes
+// and a row is sixteen heads of a token: its KV rows are copied and read from
+// LDS once for all of them, and the FP32 sequence loses the residual's terms.
+// RATIO 4: the window tile and up to eight compressed tiles, every row's HBM
+// address resident in LDS.  RATIO 1: the window tile alone.  (C128 launches
+// run c8_chunk or c8_attention.)  No explicit original slots.  STREAM:
+// non-temporal KV loads (decode-shaped launches).  ANYH: any head count up
+// to eight.
 // When graph padding leaves fewer live rows than the launch's capacity and
 // the launch may merge (`fused`: partition states and tickets supplied), the
 // live rows are re-planned with c8_attention's PLAN_FEW / PLAN_MANY rule
@@ -1524,90 +1646,72 @@ c8_merge(const SharedKVArgs p, uint32_t splits)
 // row's set-up on four waves, and one-tile partitions measured slower):
 // each work item is a (row, partition) pair, every XCD takes a contiguous
 // eighth of the live rows, and the last partition of a row folds the
-// states.  A row's tiles are a chain (QK -> tile maximum -> exponentials and
-// P codes -> PV) through work-group barriers; with one row per CU nothing
-// fills those waits, with two rows per CU the other work-group computes
-// while this one waits for its barrier or its next tile.  Each wave takes 32 keys in QK (two 16-key blocks) and 128 output
-// columns in PV.
-// RATIO 4: the window tile and up to eight compressed tiles, every row's HBM
-// address resident in LDS.  RATIO 1: the window tile alone.  (C128 launches
-// keep c8_attention: its two-tile ring keeps two tiles of a row in flight,
-// where this kernel's single buffer exposes one copy round trip per tile; on
-// C128 rows of three tiles and on joint rows that costs more than the second
-// work-group per CU gains.)
-// No explicit original slots.  STREAM: non-temporal KV copies (decode-shaped
-// launches).  ANYH: 1..128 heads, a row being one group of eight heads of a
-// token (residual codes off above eight heads, reference.py:221-222), as in
-// c8_attention.
+// states (partition states, tickets and the rule count rows of eight heads).
 constexpr int ROWS_THREADS = 256;
 constexpr int ROWS_WAVES = ROWS_THREADS / 64;
 constexpr int ROWS_TILES = 1 + MAX_LIST / N;                       // a C4 row: window tile + compressed tiles
-constexpr int ROWS_DMA = N * D / 1024 / ROWS_WAVES;               // LDS DMA instructions per wave and tile
 constexpr int ROWS_IX = MAX_LIST / ROWS_THREADS;                  // C4 index entries per thread
-static_assert(ROWS_DMA == 16 && ROWS_IX == 4, "four waves: 32 keys and 16 copies per wave and tile");
+constexpr int WIDE_HEADS = 16;
+static_assert(ROWS_IX == 4 && N / ROWS_WAVES == 32, "four waves: 32 keys, 16 loads of two rows per wave and tile");
 
 struct alignas(16) RowsShared {
-    int32_t redmax[HEADS][ROWS_WAVES];   // per-wave maxima of the tile (fkey)
-    float redsum[HEADS][ROWS_WAVES];     // per-wave sums of the wave's two 16-key blocks
-    float asc[2][HEADS];                 // alpha * softmax_scale per kind
+    int32_t redmax[WIDE_HEADS][ROWS_WAVES];   // per-wave maxima of the tile (fkey)
+    float redsum[WIDE_HEADS][ROWS_WAVES];     // per-wave sums of the wave's two 16-key blocks
+    float asc[2][WIDE_HEADS];                 // alpha * softmax_scale per kind
     int32_t scan[ROWS_WAVES];
-    int32_t misc[8];
+    int32_t misc[4];
     float scale[2][D];                   // channel scales of the window / compressed cache
-    int8_t p[16 * PROW];                 // P codes [MFMA row][key]
+    int8_t p[N * 16];                    // P codes [key][MFMA row]
     uint64_t addr[ROWS_TILES * N];       // HBM address of each row of the row's tiles (masked: the Q base)
     int8_t tile[N * D];                  // the tile buffer; Q code staging before the first tile
 };
 static_assert(sizeof(RowsShared) <= 80 * 1024, "two work-groups per CU");
-static_assert(offsetof(RowsShared, tile) % 16 == 0, "16-byte LDS DMA rows and tile reads");
+static_assert(offsetof(RowsShared, tile) % 16 == 0, "16-byte tile reads");
 
-template <int RATIO, bool STREAM, bool ANYH>
+template <int RATIO, bool STREAM, bool ANYH, bool WIDE>
 __global__ void __launch_bounds__(ROWS_THREADS, 2)
 c8_rows(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint64_t cmp_indices,
         const uint32_t batch_arg, const uint32_t topk_arg, const uint32_t rows_arg, const uint32_t grid,
         const uint32_t heads_arg, const SharedKVArgs p, const uint32_t fused)
 {
     static_assert(RATIO == 1 || RATIO == 4, "window-only and C4 launches");
+    static_assert(!WIDE || ANYH, "wide rows take any head count above eight");
+    constexpr int RH = WIDE ? WIDE_HEADS : HEADS;   // heads of a row
+    constexpr int NH = RH / 4;                      // heads of a lane group: 4 MFMA rows, {code, residual} or codes
     __shared__ RowsShared s;
-    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: copy destinations on the SALU
-    // XCD-aware order: consecutive rows stay on one XCD (their windows overlap).
-    const uint32_t G = grid;
-    // (Work-groups past the rows still take part: a re-planned launch hands
-    // out its items per XCD.)
-    const int32_t first_row = (int32_t)((blockIdx.x & 7u) * (G >> 3) + (blockIdx.x >> 3));
+    const int tid = threadIdx.x;
+    const int wave = uni(tid >> 6);
     const __attribute__((address_space(1))) int32_t *cu = gptr<int32_t>(cu_q);
     const __attribute__((address_space(1))) int32_t *lens = gptr<int32_t>(seq_lens);
     const int batch_n = (int)batch_arg, topk = RATIO == 4 ? (int)topk_arg : 0;
-
-    // ---- live shape (attention_impl.h:121-137), once per work-group ----
-    if (tid == 0) s.misc[0] = 0;
-    __syncthreads();
-    for (int b = tid; b < batch_n; b += ROWS_THREADS)
-        if (lens[b] > 0 && cu[b + 1] >= 0) atomicMax(&s.misc[0], b + 1);
-    __syncthreads();
-    const int live_batch = uni(s.misc[0]);
-    const int end = live_batch ? cu[live_batch] : 0;
-    const int live_tokens = end <= 0 ? 0 : (end < (int)p.tokens ? end : (int)p.tokens);
     const int H = ANYH ? (int)heads_arg : HEADS;                 // heads of a query token
-    const int HG = ANYH ? (H + HEADS - 1) / HEADS : 1;           // groups of eight
-    const bool resid = !ANYH || H <= HEADS;
+    const int HG = ANYH ? (H + RH - 1) / RH : 1;                 // rows of a token
+    const int HG8 = ANYH ? (H + HEADS - 1) / HEADS : 1;          // and of eight heads (the plan's rows)
+    const uint32_t G = grid;
+    const int32_t rows_cap = (int32_t)p.tokens * HG;
+    // XCD-aware order: consecutive rows stay on one XCD (their windows overlap).
+    const int32_t x = (int32_t)(blockIdx.x & 7u), slot = (int32_t)(blockIdx.x >> 3), per_xcd = (int32_t)(G >> 3);
+
+    // Every wave holds the metadata of the first 64 requests, request b in
+    // lane b, and searches them with ballots.
+    const int mine_b = (tid & 63) < batch_n ? (tid & 63) : batch_n - 1;
+    const int my_cu0 = cu[mine_b], my_cu1 = cu[mine_b + 1], my_len = lens[mine_b];
     // Channel scales: the window's, and the compressed cache's (none without one).
     if (RATIO != 1 || tid < ROWS_THREADS / 2)
         *reinterpret_cast<f32x4 *>(&s.scale[tid >> 7][(tid & 127) * 4]) =
             *gptr<f32x4>(((tid >> 7) ? p.cmpScale : p.oriScale) + (uint64_t)((tid & 127) * 4) * 4);
-    const int c0 = 128 * wave;   // this wave's PV output columns: c0 + 16 j + n
+
+    // ---- live shape (attention_impl.h:121-137) ----
+    const LiveShape live = live_shape(cu, lens, batch_n, my_cu1, my_len);
+    const int live_batch = live.batch;
+    const int live_tokens = live.end <= 0 ? 0 : (live.end < (int)p.tokens ? live.end : (int)p.tokens);
 
     // ---- device plan of a padded launch (c8_attention's rule) ----
-    const int32_t rows_cap = (int32_t)rows_arg, live_rows = live_tokens * HG;
+    const int32_t live_rows = live_tokens * HG8;
     int32_t S = 1;
-    const bool replan = fused && live_rows > 0 && live_rows < rows_cap;
+    const bool replan = fused && live_rows > 0 && live_rows < (int32_t)rows_arg;
     if (replan) {
-        if (tid == 0) s.misc[6] = 0;
-        __syncthreads();
-        for (int b = tid; b < live_batch; b += ROWS_THREADS)
-            if (lens[b] > 0 && cu[b + 1] >= 0) atomicMax(&s.misc[6], lens[b]);
-        __syncthreads();
-        const int longest = uni(s.misc[6]);
+        const int longest = longest_live(cu, lens, live_batch);
         int32_t tiles = 1;
         if (RATIO == 4) {
             const int cnt = longest / 4 < topk ? longest / 4 : topk;
@@ -1615,74 +1719,87 @@ c8_rows(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, con
         }
         int32_t plan = live_rows * PLAN_FEW <= PLAN_CUS ? PLAN_FEW : PLAN_MANY;
         const int32_t fit = PLAN_CUS / live_rows > 1 ? PLAN_CUS / live_rows : 1;
-        const int32_t room = rows_cap / live_rows;
+        const int32_t room = (int32_t)rows_arg / live_rows;
         plan = plan < fit ? plan : fit;
         plan = plan < tiles ? plan : tiles;
         plan = plan < room ? plan : room;
         S = plan > 1 ? plan : 1;
-        // Padding rows [live_rows, rows_cap) are zero (attention_impl.h:443-460).
-        for (int32_t pad = live_rows + first_row; pad < rows_cap; pad += (int32_t)G) {
-            const int32_t pt = ANYH ? pad / HG : pad, ph = ANYH ? HEADS * (pad % HG) : 0;
-            const int pl = ANYH ? (H - ph < HEADS ? H - ph : HEADS) : HEADS;
-            uint16_t *o = reinterpret_cast<uint16_t *>(p.out) + ((int64_t)pt * H + ph) * D;
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                if (!ANYH || tid + ROWS_THREADS * i < pl * (D / 8))
-                    reinterpret_cast<v4i *>(o)[tid + ROWS_THREADS * i] = v4i{0, 0, 0, 0};
-            if (p.lse && tid < pl) reinterpret_cast<float *>(p.lse)[(int64_t)pt * H + ph + tid] = 0.0f;
-        }
+        // Padding rows (attention_impl.h:443-460) are zero.
+        const int64_t words = (int64_t)p.tokens * H * (D / 8);
+        for (int64_t i = (int64_t)live_tokens * H * (D / 8) + blockIdx.x * ROWS_THREADS + tid; i < words; i += G * ROWS_THREADS)
+            reinterpret_cast<v4i *>(p.out)[i] = v4i{0, 0, 0, 0};
+        if (p.lse)
+            for (int64_t i = (int64_t)live_tokens * H + blockIdx.x * ROWS_THREADS + tid; i < (int64_t)p.tokens * H;
+                 i += G * ROWS_THREADS)
+                reinterpret_cast<float *>(p.lse)[i] = 0.0f;
     }
 
-    // Work item (query row qrow, partition part of S).
-    auto run_item = [&](const int32_t qrow, const int32_t part) {
-        const int t = ANYH ? qrow / HG : qrow;                   // token
-        const int hbase = ANYH ? HEADS * (qrow % HG) : 0;        // first head of the row
-        const int hlive = ANYH ? (H - hbase < HEADS ? H - hbase : HEADS) : HEADS;
-        uint16_t *out_row = reinterpret_cast<uint16_t *>(p.out) + ((int64_t)t * H + hbase) * D;
-        float *lse_row = p.lse ? reinterpret_cast<float *>(p.lse) + (int64_t)t * H + hbase : nullptr;
-        // Q (heads wave and wave + 4, channels 8 lane ..) and the row's index
-        // entries 4 tid .. 4 tid + 3, requested with the request search (the
-        // other work-group of the CU computes meanwhile).
-        // Q, the indices and the output are read or written once: non-temporal,
-        // so they do not displace the KV rows the launch's rows share in L2.
-        v4i qv[2];
+    // Capacity plan: rows x G / 8 + slot, + G, ...  Re-planned: the live
+    // items of this XCD, rows [x R / 8, (x + 1) R / 8) each as S partitions,
+    // over the XCD's work-groups in turn.
+    const int32_t plan_rows = live_tokens * HG;
+    const int32_t lo = replan ? x * plan_rows / 8 : 0, hi = replan ? (x + 1) * plan_rows / 8 : rows_cap;
+    const int32_t step = replan ? per_xcd : (int32_t)G;
+    int32_t item = replan ? slot : x * per_xcd + slot;
+
+    // Q (heads wave, wave + 4, ... of the row, channels 8 lane ..) and the
+    // row's index entries 4 tid .. 4 tid + 3, ahead of the row before.
+    // They and the output are read or written once: non-temporal, so they do
+    // not displace the KV rows the launch's rows share in L2.
+    v4i qv[RH / ROWS_WAVES];
+    int ix[ROWS_IX];
+    auto load_row = [&](int32_t qrow) {
+        const int t = ANYH ? qrow / HG : qrow;
+        const int hbase = ANYH ? RH * (qrow % HG) : 0;
+        const int lane = tid & 63;
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh)
-            qv[hh] = !ANYH || wave + 4 * hh < hlive
-                         ? __builtin_nontemporal_load(
-                               gptr<v4i>(q_base + (((uint64_t)t * H + hbase + wave + 4 * hh) * D + lane * 8) * 2))
-                         : v4i{0, 0, 0, 0};   // padding heads of the last group: zero Q, never written
-        int ix[ROWS_IX];
+        for (int hh = 0; hh < RH / ROWS_WAVES; ++hh) {
+            // Heads past the last read its codes again (never written).
+            int h = hbase + wave + ROWS_WAVES * hh;
+            h = !ANYH || h < H ? h : H - 1;
+            qv[hh] = __builtin_nontemporal_load(gptr<v4i>(q_base + (((uint64_t)t * H + h) * D + lane * 8) * 2));
+        }
         if (RATIO == 4) {
             const __attribute__((address_space(1))) int32_t *row_ix = gptr<int32_t>(cmp_indices) + (int64_t)t * topk;
 #pragma unroll
-            for (int e = 0; e < ROWS_IX; ++e)
-                ix[e] = tid * ROWS_IX + e < topk ? __builtin_nontemporal_load(row_ix + tid * ROWS_IX + e) : -1;
-        }
-        __syncthreads();   // every wave is done with the previous item's shared data
-        if (tid == 0) s.misc[1] = -1;
-        __syncthreads();
-        for (int b = tid; b < live_batch; b += ROWS_THREADS) {
-            const int b0 = cu[b], b1 = cu[b + 1];
-            if (b0 <= t && t < b1) {
-                s.misc[1] = b;
-                s.misc[3] = lens[b];
-                s.misc[4] = b1;
+            for (int e = 0; e < ROWS_IX; ++e) {
+                const int at = tid * ROWS_IX + e;
+                ix[e] = __builtin_nontemporal_load(row_ix + (at < topk ? at : 0));
             }
         }
-        __syncthreads();
-        const int batch = uni(s.misc[1]);
-        const int position = batch < 0 ? -1 : uni(s.misc[3]) - uni(s.misc[4]) + t;
+    };
+    if (lo + item / S >= hi) return;
+    load_row(lo + item / S);
+
+    for (bool more = true; more;) {
+        const int32_t qrow = lo + item / S, part = item % S;
+        item += step;
+        const int32_t next = lo + item / S;
+        more = next < hi;
+        // Per-lane values derive from an opaque copy of the lane index, so
+        // that none is held in a register across the rows.
+        int lane = tid & 63;
+        asm volatile("" : "+v"(lane));
+        const int g = lane >> 4, n = lane & 15;
+        const int t = ANYH ? qrow / HG : qrow;                   // token
+        const int hbase = ANYH ? RH * (qrow % HG) : 0;           // first head of the row
+        const int hlive = ANYH ? (H - hbase < RH ? H - hbase : RH) : RH;
+        uint16_t *out_row = reinterpret_cast<uint16_t *>(p.out) + ((int64_t)t * H + hbase) * D;
+        float *lse_row = p.lse ? reinterpret_cast<float *>(p.lse) + (int64_t)t * H + hbase : nullptr;
+        const Request r = find_request(cu, lens, live_batch, my_cu0, my_cu1, my_len, t);
+        const int batch = r.batch, position = batch < 0 ? -1 : r.len - r.c1 + t;
         // Padding rows of a captured graph (attention_impl.h:443-460) and rows
         // with a negative position (reference.py:104-105 rejects them) are zero.
         if (t >= live_tokens || batch < 0 || position < 0) {
-            if (part != 0) return;
+            if (part == 0) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-                if (!ANYH || tid + ROWS_THREADS * i < hlive * (D / 8))
-                    reinterpret_cast<v4i *>(out_row)[tid + ROWS_THREADS * i] = v4i{0, 0, 0, 0};
-            if (lse_row && tid < hlive) lse_row[tid] = 0.0f;
-            return;
+                for (int i = 0; i < RH / ROWS_WAVES; ++i)
+                    if (wave + ROWS_WAVES * i < hlive)
+                        reinterpret_cast<v4i *>(out_row)[64 * (wave + ROWS_WAVES * i) + lane] = v4i{0, 0, 0, 0};
+                if (lse_row && tid < hlive) lse_row[tid] = 0.0f;
+            }
+            if (more) load_row(next);
+            continue;
         }
 
         // ---- selection (attention_impl.h:58-73, reference.py:228-253) ----
@@ -1691,21 +1808,17 @@ c8_rows(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, con
         const int count = RATIO == 4 ? (position + 1) / 4 : 0;
         const __attribute__((address_space(1))) int32_t *otab = gptr<int32_t>(p.oriTable) + (int64_t)batch * p.oriTableWidth;
         const __attribute__((address_space(1))) int32_t *ctab = gptr<int32_t>(p.cmpTable) + (int64_t)batch * p.cmpTableWidth;
-        int wpage = -1, widx = -1, cpage[ROWS_IX];
-        if (tid < ori_count) {
-            const int idx = first_ori + tid;
-            if (idx / BLOCK_ROWS < (int)p.oriTableWidth) {
-                widx = idx;
-                wpage = otab[idx / BLOCK_ROWS];
-            }
-        }
-        int ipos[ROWS_IX];
+        int wpage = -1;
+        const int widx = first_ori + tid;
+        if (tid < ori_count && widx / BLOCK_ROWS < (int)p.oriTableWidth) wpage = otab[widx / BLOCK_ROWS];
+        int cpage[ROWS_IX], ipos[ROWS_IX];
         int list_len = 0;
-        bool ok[ROWS_IX];
+        lds_barrier();   // every wave is done with the previous item's shared data
         if (RATIO == 4) {
+            bool ok[ROWS_IX];
 #pragma unroll
             for (int e = 0; e < ROWS_IX; ++e) {
-                ok[e] = ix[e] >= 0 && ix[e] < count;
+                ok[e] = tid * ROWS_IX + e < topk && ix[e] >= 0 && ix[e] < count;
                 cpage[e] = ok[e] && ix[e] / BLOCK_ROWS < (int)p.cmpTableWidth ? ctab[ix[e] / BLOCK_ROWS] : -1;
             }
             // List place of each entry: compacted (count < topk <= 1024,
@@ -1733,65 +1846,100 @@ c8_rows(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, con
                 list_len = uni(total);
             } else {
 #pragma unroll
-                for (int e = 0; e < ROWS_IX; ++e) ipos[e] = ok[e] ? tid * ROWS_IX + e : -1;
+                for (int e = 0; e < ROWS_IX; ++e) ipos[e] = tid * ROWS_IX + e < topk ? tid * ROWS_IX + e : -1;
             }
         }
         const int tiles = 1 + (list_len + N - 1) / N;   // window tile, then compressed tiles
         // Tile k belongs to partition k % S (the window tile to partition 0);
         // partitions that own no tile hold the initial state, which folds to
         // nothing, and publish nothing.
-        if (part >= tiles) return;
+        if (part >= tiles) {
+            if (more) load_row(next);
+            continue;
+        }
         const int folded = S < tiles ? S : tiles;
 
         // ---- row addresses (masked rows: the Q base, never used) ----
-        for (int i = tid; i < tiles * N; i += ROWS_THREADS) s.addr[i] = p.q;
-        lds_barrier();
-        if (widx >= 0 && wpage >= 0 && (uint32_t)wpage < p.oriPages)
-            s.addr[tid] = p.ori + (uint64_t)wpage * p.oriStride + (uint64_t)((widx % BLOCK_ROWS) * D);
+        if (tid < N)
+            s.addr[tid] = (uint32_t)wpage < p.oriPages
+                              ? p.ori + (uint64_t)(uint32_t)wpage * p.oriStride + (uint64_t)((widx % BLOCK_ROWS) * D)
+                              : p.q;
         if (RATIO == 4) {
 #pragma unroll
             for (int e = 0; e < ROWS_IX; ++e)
-                if (ipos[e] >= 0 && cpage[e] >= 0)
-                    s.addr[N + ipos[e]] = p.cmp + (uint64_t)cpage[e] * p.cmpStride + (uint64_t)((ix[e] % BLOCK_ROWS) * D);
+                if (ipos[e] >= 0)
+                    s.addr[N + ipos[e]] =
+                        cpage[e] >= 0 ? p.cmp + (uint64_t)(uint32_t)cpage[e] * p.cmpStride + (uint64_t)((ix[e] % BLOCK_ROWS) * D)
+                                      : p.q;
+            if (list_len + tid < (tiles - 1) * N) s.addr[N + list_len + tid] = p.q;   // the last tile's end
         }
+        lds_barrier();
+
+        // Tile k's rows to registers: load i moves keys 32 w + i (lanes 0-31)
+        // and 32 w + 16 + i (lanes 32-63), 16 bytes a lane.
+        v4i kv[16];
+        // Quarter q of them at a time: a wave that issues all sixteen stalls
+        // behind its own queue.
+        auto fetch_rows = [&](int k, int q) {
+            typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+            const u64x2 *rows = reinterpret_cast<const u64x2 *>(s.addr + k * N + 32 * wave + 16 * (lane >> 5) + 4 * q);
+            const u64x2 ra[2] = {rows[0], rows[1]};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const auto *src = gptr<v4i>(ra[i >> 1][i & 1] + (uint64_t)((lane & 31) * 16));
+                kv[4 * q + i] = STREAM ? __builtin_nontemporal_load(src) : *src;
+            }
+        };
+        // And from there to the tile buffer.
+        auto store_tile = [&]() {
+            int lx = lane;
+            asm volatile("" : "+v"(lx));
+            lds_i8 *at = (lds_i8 *)s.tile + (32 * wave + 16 * (lx >> 5)) * D;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) *(lds_v4i *)(at + i * D + (((lx & 31) ^ i) << 4)) = kv[i];
+        };
+#pragma unroll
+        for (int q = 0; q < 4; ++q) fetch_rows(part, q);
 
         // ---- Q folding and residual split per kind (reference.py:274-279) ----
         // Staged in the tile buffer, then picked up in the MFMA A layout.
         v4i qa0[8], qa1[8];
         {
             const int want = (part == 0 ? S : part) < tiles ? 2 : 1;   // a compressed tile in this item
-            const int qe0 = lane * 8;
 #pragma unroll
             for (int kind = 0; kind < 2; ++kind) {
-                if (kind >= want) continue;
-                const float *scale = s.scale[kind] + qe0;
+                if (kind >= want || (RATIO == 1 && kind)) continue;
+                const f32x4 s0 = *reinterpret_cast<const f32x4 *>(s.scale[kind] + lane * 8);
+                const f32x4 s1 = *reinterpret_cast<const f32x4 *>(s.scale[kind] + lane * 8 + 4);
+                const float sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
-                    const int h = wave + 4 * hh;
+                for (int hh = 0; hh < RH / ROWS_WAVES; ++hh) {
+                    const int h = wave + ROWS_WAVES * hh;
                     const uint32_t qw[4] = {(uint32_t)qv[hh].x, (uint32_t)qv[hh].y, (uint32_t)qv[hh].z, (uint32_t)qv[hh].w};
                     float f[8];
                     float amax = 0.0f;
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        f[e] = bf16_to_f32((qw[e >> 1] >> (16 * (e & 1))) & 0xffffu) * scale[e];
+                        f[e] = __uint_as_float(e & 1 ? qw[e >> 1] & 0xffff0000u : qw[e >> 1] << 16) * sc[e];
                         amax = fmaxf(amax, fabsf(f[e]));
                     }
                     amax = wave_max(amax);
                     float alpha = amax * (float)(1.0 / 127.0);
                     alpha = alpha < 1e-12f ? 1e-12f : alpha;
                     const float inv = 1.0f / alpha;
-                    uint32_t hiw[2] = {0, 0}, low[2] = {0, 0};
+                    float hi8[8], lo8[8];
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        const float x = clamp127(f[e] * inv);
-                        const float hi = __builtin_rintf(x);
-                        const float lo = resid ? __builtin_rintf((x - hi) * 127.0f) : 0.0f;
-                        hiw[e >> 2] |= ((uint32_t)(int32_t)hi & 0xffu) << (8 * (e & 3));
-                        low[e >> 2] |= ((uint32_t)(int32_t)lo & 0xffu) << (8 * (e & 3));
+                        const float v = clamp127(f[e] * inv);
+                        hi8[e] = v + MAGIC;
+                        if (!WIDE) lo8[e] = (v - (hi8[e] - MAGIC)) * 127.0f + MAGIC;
                     }
-                    int8_t *stage = s.tile + kind * 16 * QSTAGE;
-                    *reinterpret_cast<u32x2 *>(stage + row_of(h, 0) * QSTAGE + qe0) = u32x2{hiw[0], hiw[1]};
-                    *reinterpret_cast<u32x2 *>(stage + row_of(h, 1) * QSTAGE + qe0) = u32x2{low[0], low[1]};
+                    int8_t *stage = s.tile + kind * 16 * QSTAGE + lane * 8;
+                    *reinterpret_cast<u32x2 *>(stage + (WIDE ? h : row_of(h, 0)) * QSTAGE) =
+                        u32x2{low_bytes(hi8[0], hi8[1], hi8[2], hi8[3]), low_bytes(hi8[4], hi8[5], hi8[6], hi8[7])};
+                    if (!WIDE)
+                        *reinterpret_cast<u32x2 *>(stage + row_of(h, 1) * QSTAGE) =
+                            u32x2{low_bytes(lo8[0], lo8[1], lo8[2], lo8[3]), low_bytes(lo8[4], lo8[5], lo8[6], lo8[7])};
                     if (lane == 0) s.asc[kind][h] = alpha * p.softmaxScale;
                 }
             }
@@ -1800,7 +1948,8 @@ c8_rows(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, con
 #pragma unroll
             for (int jj = 0; jj < 8; ++jj) {
                 qa0[jj] = *reinterpret_cast<const v4i *>(st0 + n * QSTAGE + 64 * jj + 16 * g);
-                qa1[jj] = want > 1 ? *reinterpret_cast<const v4i *>(st1 + n * QSTAGE + 64 * jj + 16 * g) : v4i{0, 0, 0, 0};
+                qa1[jj] = RATIO == 4 && want > 1 ? *reinterpret_cast<const v4i *>(st1 + n * QSTAGE + 64 * jj + 16 * g)
+                                                 : v4i{0, 0, 0, 0};
             }
             lds_barrier();   // every wave holds its Q codes: the buffer is free
         }
@@ -1808,172 +1957,186 @@ c8_rows(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, con
         // ---- tiles (reference.py:280-316 with one partition) ----
         const __attribute__((address_space(1))) float *sinks = gptr<float>(p.sinks);
         const float den0 = part == 0 ? 1.0f : 0.0f;   // the sink's exp(sink - max) starts partition 0
-        float mx[2], den[2] = {den0, den0}, num[2][8];
-        mx[0] = (!ANYH || 2 * g < hlive) ? sinks[hbase + 2 * g] : 0.0f;
-        mx[1] = (!ANYH || 2 * g + 1 < hlive) ? sinks[hbase + 2 * g + 1] : 0.0f;
+        float mx[NH], den[NH], num[NH][8];
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh)
+        for (int hh = 0; hh < NH; ++hh) {
+            const int h = NH * g + hh;
+            mx[hh] = sinks[hbase + (!ANYH || h < hlive ? h : hlive - 1)];
+            den[hh] = den0;
 #pragma unroll
             for (int j = 0; j < 8; ++j) num[hh][j] = 0.0f;
-        v4i held_acc[8];
-        float held_sc[8], held_factor[2];
-        bool held = false;
-        const uint32_t dst = (uint32_t)(uintptr_t)(lds_i8 *)(s.tile);
-        // Tile k with the Q codes of its kind: the window tile (k = 0) takes
-        // qa0, whose registers are free for the compressed tiles after it.
-        auto run_tile = [&](const int k, const v4i (&qa)[8]) {
+        }
+        // The FP32 value of a head's integers (code and residual rows, or code row).
+        auto dots_of = [&](const v4i &acc, int hh) {
+            if (WIDE) return (float)acc[hh];
+            const float dots = (float)acc[2 * hh];
+            return dots + (float)acc[2 * hh + 1] * (float)(1.0 / 127.0);
+        };
+        // LDS places of the wave's QK keys: chunk 4 j + g, and 256 bytes further
+        // chunk 16 + 4 j + g.
+        const lds_i8 *kat[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) kat[j] = (const lds_i8 *)s.tile + (32 * wave + n) * D + (((4 * j + g) ^ n) << 4);
+        // Tile k with the Q codes of its kind; then tile `ahead` is on its way.
+        auto run_tile = [&](const int k, const v4i (&qa)[8], const int ahead) {
             const int kind = k > 0 ? 1 : 0;
-            const int lane_x = lane;
-            // Copies of tile k: instruction i of wave w moves keys 16 G + r and
-            // 16 G + 8 + r (G = 2 w + i / 8, r = i % 8) into slots 16 G + 2 r
-            // and 16 G + 2 r + 1, the layout slot_of / tile_offset read.
+            store_tile();
+            if (!STREAM) __builtin_amdgcn_s_setprio(1);
+            const bool fetch_next = ahead < tiles;
+            if (fetch_next) fetch_rows(ahead, 0);
+            const int gx = g, nx = n;
+            // ---- QK: S[16 rows][32 keys of this wave] (reference.py:286-289),
+            // over the rows it stored itself: no barrier before it ----
+            v4i sacc[2] = {v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}};
             {
-                const int h = lane_x >> 5, c = lane_x & 31;
-                typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+                v4i b[2][4];
+                auto fetch = [&](int st) {   // channels 128 st .. 128 st + 127 of both key blocks
 #pragma unroll
-                for (int half = 0; half < 2; ++half) {
-                    const int grp = 2 * wave + half;
-                    const u64x2 *rows = reinterpret_cast<const u64x2 *>(s.addr + k * N + 16 * grp + 8 * h);
-                    u64x2 ra[4];
+                    for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) ra[r] = rows[r];
-                    const int hx = (h ^ grp) & 1;
+                        for (int kb = 0; kb < 2; ++kb)
+                            b[st & 1][2 * j + kb] = *(const lds_v4i *)(kat[(2 * st + j) & 3] + (st >> 1) * 256 + kb * 16 * D);
+                };
+                fetch(0);
 #pragma unroll
-                    for (int r = 0; r < 8; ++r) {
-                        const int chunk = c ^ r ^ (hx << 3);
-                        dma16<STREAM>(ra[r >> 1][r & 1] + (uint32_t)(chunk << 4),
-                                      (uint32_t)uni((int)(dst + (16 * grp + 2 * r) * D)));
-                    }
+                for (int st = 0; st < 4; ++st) {
+                    if (st + 1 < 4) fetch(st + 1);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int kb = 0; kb < 2; ++kb)
+                            sacc[kb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa[2 * st + j], b[st & 1][2 * j + kb], sacc[kb], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            if (held) {
-                // The previous tile's FP32 epilogue (reference.py:313-316) while
-                // this tile's rows are in flight.
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        float dots = (float)held_acc[j][2 * hh];
-                        dots = dots + (float)held_acc[j][2 * hh + 1] * (float)(1.0 / 127.0);
-                        const float pv = dots * held_sc[j] * (float)(1.0 / 127.0);
-                        num[hh][j] = num[hh][j] * held_factor[hh] + pv;
-                    }
-            }
-            // This wave's copies of tile k have landed.  Its QK keys are the
-            // rows it copied itself, so QK needs no barrier; the tile-maximum
-            // barrier below makes every wave's rows visible before PV.
-            vm_wait<0>();
-            // Prefill (rows from L2): the wave in its tile chain issues ahead
-            // of the other work-group's wave on the SIMD (copies, epilogue)
-            // until the tile ends.  Decode launches, bound by the stream,
-            // keep equal priority.
-            if (!STREAM) __builtin_amdgcn_s_setprio(1);
-
-            // ---- QK: S[16 rows][32 keys of this wave] (reference.py:286-289) ----
-            v4i sacc[2] = {v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}};
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                const int sl = slot_of(32 * wave + 16 * kb + n);
-                v4i b[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) b[j] = *reinterpret_cast<const v4i *>(s.tile + tile_offset(sl, 4 * j + g));
-#pragma unroll
-                for (int j = 0; j < 8; ++j) sacc[kb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa[j], b[j], sacc[kb], 0, 0, 0);
-            }
+            if (fetch_next) fetch_rows(ahead, 1);
             // ---- logits and the tile maximum (reference.py:288-303) ----
-            float lg[2][2];
+            float lg[2][NH];
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-                const bool valid = s.addr[k * N + 32 * wave + 16 * kb + n] != p.q;
+                const bool valid = s.addr[k * N + 32 * wave + 16 * kb + nx] != p.q;
 #pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
-                    float dots = (float)sacc[kb][2 * hh];
-                    dots = dots + (float)sacc[kb][2 * hh + 1] * (float)(1.0 / 127.0);
-                    const float l = dots * s.asc[kind][2 * g + hh];
+                for (int hh = 0; hh < NH; ++hh) {
+                    float l = dots_of(sacc[kb], hh) * s.asc[kind][NH * gx + hh];
+                    asm volatile("" : "+v"(l));   // a select, not a branch
                     lg[kb][hh] = valid ? l : -1e30f;
                 }
             }
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
+            for (int hh = 0; hh < NH; ++hh) {
                 const int kmax = row16_max_key(max(fkey(lg[0][hh]), fkey(lg[1][hh])));
-                if (n == 0) s.redmax[2 * g + hh][wave] = kmax;
+                if (nx == 0) s.redmax[NH * gx + hh][wave] = kmax;
             }
             lds_barrier();
-            float mnew[2], factor[2];
+            if (fetch_next) fetch_rows(ahead, 2);
+            float mnew[NH], factor[NH];
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                const v4i a = *reinterpret_cast<const v4i *>(&s.redmax[2 * g + hh][0]);
+            for (int hh = 0; hh < NH; ++hh) {
+                const v4i a = *reinterpret_cast<const v4i *>(&s.redmax[NH * gx + hh][0]);
                 mnew[hh] = fkey_value(max(max(fkey(mx[hh]), a.x), max(max(a.y, a.z), a.w)));
             }
             {
-                const bool odd = n & 1;   // exp(max_old - max_new), one exponential per lane pair
-                const float mine = sk_expf_nonpos(odd ? mx[1] - mnew[1] : mx[0] - mnew[0]);
-                const float other = dpp<DPP_XOR1>(mine);
-                factor[0] = odd ? other : mine;
-                factor[1] = odd ? mine : other;
+                // exp(max_old - max_new): one exponential per lane, head n % NH
+                // of the group, handed round its quad.
+                const int q = nx & (NH - 1);
+                float d = mx[0] - mnew[0];
+#pragma unroll
+                for (int hh = 1; hh < NH; ++hh) d = q == hh ? mx[hh] - mnew[hh] : d;
+                const float mine = sk_expf_nonpos(d);
+                if (WIDE) {
+                    factor[0] = dpp<0x00>(mine);
+                    factor[1] = dpp<0x55>(mine);
+                    factor[NH - 2] = dpp<0xAA>(mine);
+                    factor[NH - 1] = dpp<0xFF>(mine);
+                } else {
+                    factor[0] = dpp<0xA0>(mine);   // lanes 0, 0, 2, 2
+                    factor[1] = dpp<0xF5>(mine);   // lanes 1, 1, 3, 3
+                }
             }
             // ---- weights, pairwise tile sum, P codes (reference.py:304-312) ----
-            float wsum[2];
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                float blk[2];
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb) {
-                    const int key = 32 * wave + 16 * kb + n;
-                    const float w = sk_expf_nonpos(lg[kb][hh] - mnew[hh]);
-                    const float x = w * 127.0f;
-                    const float ph = __builtin_rintf(x);
-                    const float pl = resid ? __builtin_rintf((x - ph) * 127.0f) : 0.0f;
-                    s.p[row_of(2 * g + hh, 0) * PROW + key] = (int8_t)(int32_t)ph;
-                    s.p[row_of(2 * g + hh, 1) * PROW + key] = (int8_t)(int32_t)pl;
-                    blk[kb] = row16_tree_sum(w);   // one 16-key block
-                }
-                wsum[hh] = blk[0] + blk[1];        // blocks 2 w and 2 w + 1
-                if (n == 0) s.redsum[2 * g + hh][wave] = wsum[hh];
-            }
-            lds_barrier();
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                const f32x4 a = *reinterpret_cast<const f32x4 *>(&s.redsum[2 * g + hh][0]);
-                const float tile_sum = (a.x + a.y) + (a.z + a.w);   // pairwise over the eight blocks
-                den[hh] = den[hh] * factor[hh] + tile_sum;
-            }
-            // ---- PV: [16 rows][this wave's 128 columns] (reference.py:310-316) ----
-            v4i vacc[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) vacc[j] = v4i{0, 0, 0, 0};
-            const lds_i8 *vbase = (const lds_i8 *)(s.tile);
+            float blk[2][NH];
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-                const v4i pa = *reinterpret_cast<const v4i *>(s.p + n * PROW + 64 * kb + 16 * g);
-                const int sl_lo = slot_of(64 * kb + 16 * g + (n >> 1));
-                const int sl_hi = slot_of(64 * kb + 16 * g + 8 + (n >> 1));
+                float code[4];
 #pragma unroll
-                for (int jh = 0; jh < 2; ++jh) {
-                    v2i b0[4], b1[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int chunk = 8 * wave + 4 * jh + j;
-                        b0[j] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(vbase + tile_offset(sl_lo, chunk) + 8 * (n & 1)));
-                        b1[j] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(vbase + tile_offset(sl_hi, chunk) + 8 * (n & 1)));
+                for (int hh = 0; hh < NH; ++hh) {
+                    const float w = sk_expf_nonpos(lg[kb][hh] - mnew[hh]);
+                    const float xw = w * 127.0f;
+                    if (WIDE) {
+                        code[hh] = xw + MAGIC;
+                    } else {
+                        code[2 * hh] = xw + MAGIC;
+                        code[2 * hh + 1] = (xw - (code[2 * hh] - MAGIC)) * 127.0f + MAGIC;
                     }
+                    blk[kb][hh] = row16_tree_sum(w);   // one 16-key block
+                }
+                *(lds_u32 *)((lds_i8 *)s.p + (32 * wave + 16 * kb + nx) * 16 + 4 * gx) = low_bytes(code[0], code[1], code[2], code[3]);
+            }
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const v4i vb = {b0[j].x, b0[j].y, b1[j].x, b1[j].y};
-                        vacc[4 * jh + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(pa, vb, vacc[4 * jh + j], 0, 0, 0);
+            for (int hh = 0; hh < NH; ++hh)
+                if (nx == 0) s.redsum[NH * gx + hh][wave] = blk[0][hh] + blk[1][hh];   // blocks 2 w and 2 w + 1
+            lds_barrier();
+            if (fetch_next) fetch_rows(ahead, 3);
+#pragma unroll
+            for (int hh = 0; hh < NH; ++hh) {
+                const f32x4 a = *reinterpret_cast<const f32x4 *>(&s.redsum[NH * gx + hh][0]);
+                const float tile_sum = (a.x + a.y) + (a.z + a.w);   // pairwise over the eight blocks
+                den[hh] = den[hh] * factor[hh] + tile_sum;
+                mx[hh] = mnew[hh];
+            }
+            // ---- PV: [16 rows][this wave's 128 columns] (reference.py:310-316),
+            // two 16-column blocks at a time, each followed by its FP32 epilogue ----
+            {
+                v4i pa[2];
+                const lds_i8 *pat = (const lds_i8 *)s.p + (8 * gx + (nx >> 1)) * 16 + 8 * (nx & 1);
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) {
+                    const v2i a = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(pat + kb * 1024));
+                    const v2i b = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(pat + kb * 1024 + 512));
+                    pa[kb] = v4i{a.x, a.y, b.x, b.y};
+                }
+                const float *sc = s.scale[kind] + 128 * wave + nx;
+                int lx = lane;
+                if (WIDE) asm volatile("" : "+v"(lx));   // (wide rows have no registers to hold these across the tiles)
+                const int vr = 8 * (lx >> 4) + ((lx & 15) >> 1);   // V row of the lane's reads
+                const lds_i8 *vat[8];
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+                    vat[c] = (const lds_i8 *)s.tile + vr * D + 8 * (lx & 1) + (wave >> 1) * 256 + (((8 * (wave & 1) + c) ^ (vr & 15)) << 4);
+                v2i bb[2][8];
+                auto fetch = [&](int jc) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const lds_i8 *cat = vat[2 * jc + j];
+#pragma unroll
+                        for (int kb = 0; kb < 2; ++kb) {
+                            bb[jc & 1][4 * j + 2 * kb] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(cat + kb * 64 * D));
+                            bb[jc & 1][4 * j + 2 * kb + 1] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(cat + kb * 64 * D + 32 * D));
+                        }
                     }
+                };
+                fetch(0);
+#pragma unroll
+                for (int jc = 0; jc < 4; ++jc) {
+                    if (jc + 1 < 4) fetch(jc + 1);
+                    v4i acc[2] = {v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}};
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) {
+                            const v2i a = bb[jc & 1][4 * j + 2 * kb], b = bb[jc & 1][4 * j + 2 * kb + 1];
+                            acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(pa[kb], v4i{a.x, a.y, b.x, b.y}, acc[j], 0, 0, 0);
+                        }
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const float scale = sc[16 * (2 * jc + j)];
+#pragma unroll
+                        for (int hh = 0; hh < NH; ++hh)
+                            num[hh][2 * jc + j] = num[hh][2 * jc + j] * factor[hh] + dots_of(acc[j], hh) * scale * (float)(1.0 / 127.0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                held_acc[j] = vacc[j];
-                held_sc[j] = s.scale[kind][c0 + 16 * j + n];
-            }
-            held_factor[0] = factor[0];
-            held_factor[1] = factor[1];
-            held = true;
-            mx[0] = mnew[0];
-            mx[1] = mnew[1];
             if (!STREAM) __builtin_amdgcn_s_setprio(0);
             lds_barrier();   // every wave is done with tile k and the P codes
         };
@@ -1983,43 +2146,48 @@ c8_rows(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, con
             v4i qf[8];
 #pragma unroll
             for (int jj = 0; jj < 8; ++jj) qf[jj] = part == 0 ? qa0[jj] : qa1[jj];
-            run_tile(part, qf);
+            run_tile(part, qf, RATIO == 4 ? part + S : tiles);
         }
-        for (int k = part + S; k < tiles; k += S) run_tile(k, qa1);
-        if (held) {
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    float dots = (float)held_acc[j][2 * hh];
-                    dots = dots + (float)held_acc[j][2 * hh + 1] * (float)(1.0 / 127.0);
-                    const float pv = dots * held_sc[j] * (float)(1.0 / 127.0);
-                    num[hh][j] = num[hh][j] * held_factor[hh] + pv;
-                }
+        if (RATIO == 4) {
+#pragma nounroll
+            for (int k = part + S; k < tiles; k += S) run_tile(k, qa1, k + S);
         }
+        if (more) load_row(next);
+        const int c0 = 128 * wave;   // this wave's PV output columns: c0 + 16 j + n
         if (folded == 1) {
             // ---- finalize (reference.py:317-323 with one partition) ----
+            const uint32_t pick = n & 1 ? 0x03020706u : 0x05040100u;
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                const int h = 2 * g + hh;
-                if (ANYH && h >= hlive) continue;
+            for (int hh = 0; hh < NH; ++hh) {
+                const int h = NH * g + hh;
+                const float rden = 1.0f / den[hh];
+                uint32_t *to = reinterpret_cast<uint32_t *>(out_row + h * D + c0) + 8 * (n & 1) + (n >> 1);
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    __builtin_nontemporal_store((uint16_t)pack_bf16(num[hh][j] / den[hh], 0.0f), out_row + h * D + c0 + 16 * j + n);
-                if (lse_row && wave == 0 && n == 0) lse_row[h] = mx[hh] + logf(den[hh]);
+                for (int j = 0; j < 8; j += 2) {
+                    // Lanes n and n ^ 1 exchange one column of two, so that each writes two neighbours.
+                    const uint32_t mine = pack_bf16(div_by(num[hh][j], den[hh], rden), div_by(num[hh][j + 1], den[hh], rden));
+                    const uint32_t other = (uint32_t)dpp_i<DPP_XOR1>((int)mine);
+                    const uint32_t both = __builtin_amdgcn_perm(other, mine, pick);
+                    if (!ANYH || h < hlive) __builtin_nontemporal_store(both, to + 8 * j);
+                }
+                if (lse_row && wave == 0 && n == 0 && (!ANYH || h < hlive)) lse_row[h] = mx[hh] + logf(den[hh]);
             }
-            return;
+            continue;
         }
         // ---- publish this partition, the last one to finish folds the row
         // (the protocol of c8_attention's fused merge; a re-planned row's
         // partitions all run on one XCD, so with the XCD-local exchange its
-        // states pass through that XCD's L2) ----
+        // states pass through that XCD's L2).  States and tickets are those
+        // of rows of eight heads ----
         const bool local = (fused & FUSED_XCD_LOCAL) != 0;
-        const __amdgpu_buffer_rsrc_t states =
-            row_states(reinterpret_cast<float *>(p.partial) + (int64_t)qrow * S * HEADS * PART_FLOATS);
+        const int row8 = WIDE ? t * HG8 + 2 * (qrow % HG) : qrow, groups = WIDE && hlive > HEADS ? 2 : 1;
+        float *partial = reinterpret_cast<float *>(p.partial);
+        const __amdgpu_buffer_rsrc_t states = row_states(partial + (int64_t)row8 * S * HEADS * PART_FLOATS);
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            const int base = ((part * HEADS + 2 * g + hh) * PART_FLOATS) * 4;
+        for (int hh = 0; hh < NH; ++hh) {
+            const int h = NH * g + hh;
+            if (WIDE && h >= groups * HEADS) continue;
+            const int base = (((h / HEADS) * S * HEADS + part * HEADS + h % HEADS) * PART_FLOATS) * 4;
             if (local) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) state_store<SC0>(num[hh][j], states, base + (c0 + 16 * j + n) * 4);
@@ -2040,28 +2208,24 @@ c8_rows(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, con
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         uint32_t *tickets = reinterpret_cast<uint32_t *>(p.workspace);
-        if (tid == 0) s.misc[5] = (int)__hip_atomic_fetch_add(&tickets[qrow], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0) s.misc[0] = (int)__hip_atomic_fetch_add(&tickets[row8], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
-        if (s.misc[5] != folded - 1) return;
-        if (tid == 0) __hip_atomic_store(&tickets[qrow], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (s.misc[0] != folded - 1) continue;
+        if (tid == 0) __hip_atomic_store(&tickets[row8], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         // fold_row covers eight heads with 512 threads: heads 0-3, then 4-7
-        // (one copy of its code: the loop is kept).
+        // of each group (one copy of its code: the loop is kept).
 #pragma nounroll
-        for (int half = 0; half < 2; ++half) {
-            if (local) fold_row<SC0>(states, folded, tid + ROWS_THREADS * half, out_row, lse_row, ANYH ? hlive : HEADS);
-            else fold_row<SC1>(states, folded, tid + ROWS_THREADS * half, out_row, lse_row, ANYH ? hlive : HEADS);
+        for (int half = 0; half < 2 * groups; ++half) {
+            const int gr = half >> 1;
+            const __amdgpu_buffer_rsrc_t at = row_states(partial + (int64_t)(row8 + gr) * S * HEADS * PART_FLOATS);
+            uint16_t *to = out_row + gr * HEADS * D;
+            float *lse_to = lse_row ? lse_row + gr * HEADS : nullptr;
+            const int heads = ANYH ? (hlive - gr * HEADS < HEADS ? hlive - gr * HEADS : HEADS) : HEADS;
+            if (local) fold_row<SC0>(at, folded, tid + ROWS_THREADS * (half & 1), to, lse_to, heads);
+            else fold_row<SC1>(at, folded, tid + ROWS_THREADS * (half & 1), to, lse_to, heads);
         }
-    };
-
-    // Capacity plan: rows first_row, first_row + G, ...  Re-planned: the live
-    // items of this XCD, rows [x R / 8, (x + 1) R / 8) each as S partitions,
-    // over the XCD's work-groups in turn.
-    const int32_t x = (int32_t)(blockIdx.x & 7u);
-    const int32_t lo = replan ? x * live_rows / 8 : 0, hi = replan ? (x + 1) * live_rows / 8 : rows_cap;
-    const int32_t step = replan ? (int32_t)(G >> 3) : (int32_t)G;
-    for (int32_t j = replan ? (int32_t)(blockIdx.x >> 3) : first_row; lo + j / S < hi; j += step)
-        run_item(lo + j / S, j % S);
+    }
 }
 
 // ---- c8_pairs: query-grouped plans (groups of two or four query tokens) ----
@@ -2809,8 +2973,6 @@ c8_pairs(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
 // T = 2048, C128 at 8 K / 32 K / 128 K context 62 / 79 / 160 -> 27 / 33 / 69
 // us, window-only 26 -> 17; T = 4096 C128 at 32 K 156 -> 62, window-only
 // 48 -> 32.
-typedef __attribute__((address_space(3))) v4i lds_v4i;
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
 constexpr int CHUNK_ROWS = 8;                        // query rows of a work-group (one per wave)
 constexpr int CHUNK_UNION = N + CHUNK_ROWS;          // window rows of an octet (135 at most), in pairs
 constexpr int OUT_STRIDE = 2 * D + 32;               // LDS row stride of a head's BF16 output
@@ -2824,28 +2986,6 @@ struct alignas(16) ChunkShared {
 };
 static_assert(sizeof(ChunkShared) <= 160 * 1024, "one work-group per CU");
 static_assert(CHUNK_ROWS * HEADS * OUT_STRIDE <= CHUNK_UNION * D, "output staging fits one buffer");
-
-// x rounded to the nearest even integer sits in the low bits of x + MAGIC
-// (|x| < 2^22), so the low byte of the sum is the INT8 code.
-constexpr float MAGIC = 12582912.0f;
-__device__ __forceinline__ uint32_t low_bytes(float a, float b, float c, float d)
-{
-    const uint32_t ab = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x0c0c0400u);
-    const uint32_t cd = __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(c), 0x04000c0cu);
-    return ab | cd;
-}
-
-// num / den, correctly rounded, from the correctly rounded reciprocal r of
-// den: the FMA residual of the product corrects it (Markstein, 1990; den is
-// a softmax denominator, so no operand is subnormal).
-__device__ __forceinline__ float div_by(float num, float den, float r)
-{
-    const float q = num * r;
-    // An infinite quotient's residual is NaN; the median turns that into a
-    // finite number, which leaves the infinity as it is.
-    const float e = __builtin_amdgcn_fmed3f(__builtin_fmaf(-q, den, num), -3.0e38f, 3.0e38f);
-    return __builtin_fmaf(e, r, q);
-}
 
 // LDS DMA of 16 bytes per lane from a scalar base and a 32-bit lane offset.
 #pragma clang diagnostic push
@@ -2917,48 +3057,10 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
     load_row();
 
     // ---- live shape (attention_impl.h:121-137) ----
-    // The last request with seq_len > 0 and cu_q >= 0 ends the live batch;
-    // its cu_q end bounds the live tokens.
-    int live_batch = 0, end = 0;
-    {
-        const uint64_t there = __ballot((tid & 63) < batch_n && my_len > 0 && my_cu1 >= 0);
-        if (there) {
-            const int b = 63 - __builtin_clzll(there);
-            live_batch = b + 1;
-            end = __builtin_amdgcn_readlane(my_cu1, b);
-        }
-        for (int b0 = 64; b0 < batch_n; b0 += 64) {
-            const int b = b0 + (tid & 63) < batch_n ? b0 + (tid & 63) : batch_n - 1;
-            const int c1 = cu[b + 1];
-            const uint64_t more = __ballot(b == b0 + (tid & 63) && lens[b] > 0 && c1 >= 0);
-            if (more) {
-                live_batch = b0 + 64 - __builtin_clzll(more);
-                end = __builtin_amdgcn_readlane(c1, 63 - __builtin_clzll(more));
-            }
-        }
-    }
-    const int live_tokens = end <= 0 ? 0 : (end < (int)p.tokens ? end : (int)p.tokens);
-    // The request holding `token` (batch < 0: none), as batch, cu[b], cu[b + 1], len.
-    struct Request { int batch, c0, c1, len; };
-    auto find_request = [&](int token) {
-        const uint64_t hit = __ballot((tid & 63) < live_batch && my_cu0 <= token && token < my_cu1);
-        if (hit) {
-            const int b = __builtin_ctzll(hit);
-            return Request{b, __builtin_amdgcn_readlane(my_cu0, b), __builtin_amdgcn_readlane(my_cu1, b),
-                           __builtin_amdgcn_readlane(my_len, b)};
-        }
-        for (int b0 = 64; b0 < live_batch; b0 += 64) {
-            const int b = b0 + (tid & 63) < live_batch ? b0 + (tid & 63) : live_batch - 1;
-            const int c0 = cu[b], c1 = cu[b + 1], len = lens[b];
-            const uint64_t more = __ballot(c0 <= token && token < c1);
-            if (more) {
-                const int at = __builtin_ctzll(more);
-                return Request{b0 + at < live_batch ? b0 + at : live_batch - 1, __builtin_amdgcn_readlane(c0, at),
-                               __builtin_amdgcn_readlane(c1, at), __builtin_amdgcn_readlane(len, at)};
-            }
-        }
-        return Request{-1, 0, 0, 0};
-    };
+    const LiveShape live = live_shape(cu, lens, batch_n, my_cu1, my_len);
+    const int live_batch = live.batch;
+    const int live_tokens = live.end <= 0 ? 0 : (live.end < (int)p.tokens ? live.end : (int)p.tokens);
+    auto request_of = [&](int token) { return find_request(cu, lens, live_batch, my_cu0, my_cu1, my_len, token); };
     lds_i8 *const buf = (lds_i8 *)s.buf[0], *const pw = (lds_i8 *)s.p[0] + wave * N * 16;
     auto zero_row = [&](int t, int hbase, int hlive) {
         const int lane = tid & 63;
@@ -2978,14 +3080,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
             // partitions each (its rule, c8_attention.device_splits on the
             // host, over this launch's work-groups), unless every row is a
             // joint row.
-            int longest = 0;
-            for (int b0 = 0; b0 < live_batch; b0 += 64) {
-                const int b = b0 + (tid & 63) < live_batch ? b0 + (tid & 63) : live_batch - 1;
-                int len = cu[b + 1] >= 0 ? lens[b] : 0;
-#pragma unroll
-                for (int d = 1; d < 64; d *= 2) len = max(len, __shfl_xor(len, d));
-                longest = max(longest, uni(len));
-            }
+            const int longest = longest_live(cu, lens, live_batch);
             const int live_rows = live_tokens * HG, tiles = 1 + (longest / RATIO + N - 1) / N;
             if (tiles > 1 && PLAN_CUS / live_rows > 1 && !(resid && longest / RATIO <= N)) {
                 attention_item<RATIO, false, false, ANYH, false, true>(
@@ -3058,7 +3153,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
         tail = true;
         o = first * HG / CHUNK_ROWS;
         load_row();
-        const int c1 = find_request(first).c1;
+        const int c1 = request_of(first).c1;
         stop = c1 < stop ? c1 : stop;
         return true;
     };
@@ -3089,7 +3184,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
             const int g = lane >> 4, n = lane & 15;
             // Tokens of no live request and negative positions (reference.py:
             // 104-105 rejects them) are zero.
-            const Request r0 = find_request(first);
+            const Request r0 = request_of(first);
             if (r0.batch < 0 || r0.len - r0.c1 + first < 0) {
                 if (t == first) zero_row(t, hbase, hlive);
                 ++first;
@@ -3121,7 +3216,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
             // row needs its window and its tile together).
             bool two = false;
             if (!split && past[0] < stop && past[0] < live_tokens) {
-                const Request r1 = find_request(past[0]);
+                const Request r1 = request_of(past[0]);
                 if (r1.batch >= 0 && r1.len - r1.c1 + past[0] >= 0) {
                     segment(1, past[0], r1);
                     auto may_join = [&](int i) { return (back[i] + from[i] + 1) / RATIO <= N && all_rows[i] > 0; };
@@ -3732,7 +3827,8 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
     }
     // One-partition C4 and window-only launches of more rows than CUs
     // (prefill, large decode batches) without explicit slots run two
-    // four-wave work-groups per CU taking rows in turn (c8_rows).  Other C128
+    // four-wave work-groups per CU taking rows in turn (c8_rows; above eight
+    // heads rows of sixteen).  Other C128
     // launches keep one work-group per row: c8_attention's two-tile ring
     // measured faster on them (decode of 512 rows 51 against 72 us).
     const bool persist = !DEBUG && !slots && splits == 1 && rows > (uint32_t)PLAN_CUS &&
@@ -3740,10 +3836,21 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
     if (persist) {
         // Two four-wave work-groups per CU (c8_rows), at most one per row, so
         // that every XCD gets its share of the rows.
-        const uint32_t g2 = rows < 2u * (uint32_t)PLAN_CUS ? (rows + 7u) & ~7u : 2u * (uint32_t)PLAN_CUS;
-        const auto rows_kernel = a->ratio == 1 ? &c8_rows<1, false, ANYH>
-                                 : streamed    ? &c8_rows<4, true, ANYH>
-                                               : &c8_rows<4, false, ANYH>;
+        // Above eight heads a row of the kernel is sixteen heads of a token.
+        // (Launches of at most PLAN_CUS rows of eight heads stay on
+        // c8_attention: 256 rows, 32 sequences of 64 heads, take 23 us there,
+        // their 128 wide rows 32 us here.)
+        const uint32_t wide = ANYH && a->heads > HEADS;
+        const uint32_t own = wide ? a->tokens * ((a->heads + WIDE_HEADS - 1) / WIDE_HEADS) : rows;
+        const uint32_t g2 = own < 2u * (uint32_t)PLAN_CUS ? (own + 7u) & ~7u : 2u * (uint32_t)PLAN_CUS;
+        auto rows_kernel = a->ratio == 1 ? &c8_rows<1, false, ANYH, false>
+                           : streamed    ? &c8_rows<4, true, ANYH, false>
+                                         : &c8_rows<4, false, ANYH, false>;
+        if constexpr (ANYH)
+            if (wide)
+                rows_kernel = a->ratio == 1 ? &c8_rows<1, false, true, true>
+                              : streamed    ? &c8_rows<4, true, true, true>
+                                            : &c8_rows<4, false, true, true>;
         hipLaunchKernelGGL(rows_kernel, dim3(g2), dim3(ROWS_THREADS), 0, stream, a->cuQ, a->seqLens, a->q, a->indices,
                            a->batch, a->topk, rows, g2, a->heads, *a, fused);
         return;
