@@ -68,7 +68,6 @@ constexpr int N = SHAREDKV_C8_TILE;    // keys per tile
 constexpr int32_t PLAN_CUS = 256, PLAN_FEW = 5, PLAN_MANY = 3, PLAN_ONE_TILE = 112;
 constexpr int THREADS = 512;           // 8 waves: two per SIMD
 constexpr int WAVES = THREADS / 64;
-constexpr int PROW = N + 16;           // LDS row stride of the P codes
 constexpr int CODE_TILES = 12;         // tiles whose row codes are resident at once
 constexpr int MAX_LIST = 1024;         // C4 top-k capacity of the index list
 constexpr int PART_FLOATS = 520;       // per (row, split, head): 512 numerator, max, denominator
@@ -282,13 +281,48 @@ struct alignas(16) Shared {
     int32_t mult[N];                // joint C4 rows: multiplicity of compressed row r among the top-k entries
     float bias[N];                  // joint C4 rows: log(multiplicity) of compressed list position j
     float scale[2][D];              // channel scales of the window / compressed cache
-    int8_t p[16 * PROW];            // P codes [MFMA row][key]
+    int8_t p[16 * N];               // P codes [key][MFMA row]
     int32_t code[CODE_TILES * N];   // row codes of the resident tiles: page * 32 + row, -1 masked
     uint64_t addr[CODE_TILES * N];  // HBM address of each resident row (masked rows: an in-bounds dummy)
     int8_t tile[2][N * D];          // two K/V tiles (the DMA ring); Q code staging before the first tile
 };
 static_assert(2 * 16 * QSTAGE <= N * D, "Q staging fits in one tile buffer");
 static_assert(offsetof(Shared, tile) % 16 == 0, "16-byte LDS DMA rows and tile reads");
+
+typedef __attribute__((address_space(3))) v4i lds_v4i;
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+// x rounded to the nearest even integer sits in the low bits of x + MAGIC
+// (|x| < 2^22), so the low byte of the sum is the INT8 code.
+constexpr float MAGIC = 12582912.0f;
+__device__ __forceinline__ uint32_t low_bytes(float a, float b, float c, float d)
+{
+    const uint32_t ab = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x0c0c0400u);
+    const uint32_t cd = __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(c), 0x04000c0cu);
+    return ab | cd;
+}
+
+// num / den, correctly rounded, from the correctly rounded reciprocal r of
+// den: the FMA residual of the product corrects it (Markstein, 1990; den is
+// a softmax denominator, so no operand is subnormal).
+__device__ __forceinline__ float div_by(float num, float den, float r)
+{
+    const float q = num * r;
+    // An infinite quotient's residual is NaN; the median turns that into a
+    // finite number, which leaves the infinity as it is.
+    const float e = __builtin_amdgcn_fmed3f(__builtin_fmaf(-q, den, num), -3.0e38f, 3.0e38f);
+    return __builtin_fmaf(e, r, q);
+}
+
+// P codes of keys 64 kb + 16 g .. + 15 in the MFMA A layout, from a tile's
+// key-major codes (16 bytes a key, one 32-bit write per lane and key where
+// row-major codes take four byte writes).
+__device__ __forceinline__ v4i codes_of(const lds_i8 *p, int kb, int g, int n)
+{
+    const lds_i8 *at = p + (64 * kb + 16 * g + (n >> 1)) * 16 + 8 * (n & 1);
+    const v2i a = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)at);
+    const v2i b = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(at + 8 * 16));
+    return v4i{a.x, a.y, b.x, b.y};
+}
 
 struct Row {
     int32_t batch, position, first_ori, ori_count, count, list_len, t0, total;
@@ -379,9 +413,10 @@ __device__ __forceinline__ void fold_states(const __amdgpu_buffer_rsrc_t states,
             acc[6] = acc[6] + v1[sp].z * f[sp];
             acc[7] = acc[7] + v1[sp].w * f[sp];
         }
+    const float r = 1.0f / dsum;
     uint32_t w[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = pack_bf16(acc[2 * e] / dsum, acc[2 * e + 1] / dsum);
+    for (int e = 0; e < 4; ++e) w[e] = pack_bf16(div_by(acc[2 * e], dsum, r), div_by(acc[2 * e + 1], dsum, r));
     if (heads < HEADS && h >= heads) return;   // padding heads of the last group of eight
     *reinterpret_cast<v4i *>(out_row + h * D + col) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     if (lse_row && (tid & 63) == 0) lse_row[h] = top + logf(dsum);
@@ -438,9 +473,10 @@ __device__ __forceinline__ void fold_states_wide(const __amdgpu_buffer_rsrc_t st
                 acc[7] = acc[7] + v1[k].w * f;
             }
     }
+    const float r = 1.0f / dsum;
     uint32_t w[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = pack_bf16(acc[2 * e] / dsum, acc[2 * e + 1] / dsum);
+    for (int e = 0; e < 4; ++e) w[e] = pack_bf16(div_by(acc[2 * e], dsum, r), div_by(acc[2 * e + 1], dsum, r));
     if (heads < HEADS && h >= heads) return;
     *reinterpret_cast<v4i *>(out_row + h * D + col) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     if (lse_row && (tid & 63) == 0) lse_row[h] = top + logf(dsum);
@@ -471,7 +507,7 @@ __device__ __forceinline__ void fold_row(const __amdgpu_buffer_rsrc_t states, in
 // (reference.py:221-222: residual quantization only for <= 8 heads), which
 // leaves every other operation as it is.  Without ANYH, heads == 8.
 // The work of one work-group: item `item` of the launch's `items`.
-template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT>
+template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT, bool RESID>
 __device__ __forceinline__ void
 attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint64_t cmp_indices,
                const uint32_t batch_arg, const uint32_t topk_arg, const uint32_t heads_arg, const uint32_t splits,
@@ -488,7 +524,7 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
     if (item >= items) return;
     const int H = ANYH ? (int)heads_arg : HEADS;                 // heads of a query token
     const int HG = ANYH ? (H + HEADS - 1) / HEADS : 1;           // groups of eight
-    const bool resid = !ANYH || H <= HEADS;
+    constexpr bool resid = RESID;
     // The launch's plan: `splits` partitions per row over rows_arg rows.
     // rows.  The work item's row under that plan is loaded at once; with
     // graph padding the device re-plans (below) and may move it.
@@ -863,7 +899,7 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     float dots = (float)held_acc[j][2 * hh];
-                    dots = dots + (float)held_acc[j][2 * hh + 1] * (float)(1.0 / 127.0);
+                    if (resid) dots = dots + (float)held_acc[j][2 * hh + 1] * (float)(1.0 / 127.0);
                     const float pv = dots * held_sc[j] * (float)(1.0 / 127.0);
                     num[hh][j] = num[hh][j] * held_factor[hh] + pv;
                 }
@@ -896,22 +932,22 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
                 float amax = 0.0f;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    f[e] = bf16_to_f32((qw[e >> 1] >> (16 * (e & 1))) & 0xffffu) * scale[e];
+                    f[e] = __uint_as_float(e & 1 ? qw[e >> 1] & 0xffff0000u : qw[e >> 1] << 16) * scale[e];
                     amax = fmaxf(amax, fabsf(f[e]));
                 }
                 amax = wave_max(amax);              // the head's 512 channels
                 float alpha = amax * (float)(1.0 / 127.0);
                 alpha = alpha < 1e-12f ? 1e-12f : alpha;
                 const float inv = 1.0f / alpha;
-                uint32_t hiw[2] = {0, 0}, low[2] = {0, 0};
+                float hi[8], lo[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const float x = clamp127(f[e] * inv);
-                    const float hi = __builtin_rintf(x);
-                    const float lo = resid ? __builtin_rintf((x - hi) * 127.0f) : 0.0f;
-                    hiw[e >> 2] |= ((uint32_t)(int32_t)hi & 0xffu) << (8 * (e & 3));
-                    low[e >> 2] |= ((uint32_t)(int32_t)lo & 0xffu) << (8 * (e & 3));
+                    hi[e] = x + MAGIC;
+                    lo[e] = resid ? (x - (hi[e] - MAGIC)) * 127.0f + MAGIC : 0.0f;
                 }
+                const uint32_t hiw[2] = {low_bytes(hi[0], hi[1], hi[2], hi[3]), low_bytes(hi[4], hi[5], hi[6], hi[7])};
+                const uint32_t low[2] = {low_bytes(lo[0], lo[1], lo[2], lo[3]), low_bytes(lo[4], lo[5], lo[6], lo[7])};
                 int8_t *stage = s.tile[1] + kind * 16 * QSTAGE;
                 *reinterpret_cast<u32x2 *>(stage + row_of(wave, 0) * QSTAGE + qe0) = u32x2{hiw[0], hiw[1]};
                 *reinterpret_cast<u32x2 *>(stage + row_of(wave, 1) * QSTAGE + qe0) = u32x2{low[0], low[1]};
@@ -1174,21 +1210,21 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
                 // Weights and P codes (reference.py:194-198); the compressed
                 // tile's P codes go to the free address table.
                 int8_t *p1 = reinterpret_cast<int8_t *>(s.addr);
-                static_assert(16 * PROW <= (int)sizeof(s.addr), "P codes of the second tile fit the address table");
+                static_assert(16 * N <= (int)sizeof(s.addr), "P codes of the second tile fit the address table");
 #pragma unroll
                 for (int kind = 0; kind < 2; ++kind) {
                     int8_t *pk = kind ? p1 : s.p;
+                    float code[4];
 #pragma unroll
                     for (int hh = 0; hh < 2; ++hh) {
                         const float w = sk_expf_nonpos(lg[kind][hh] - mnew[hh]);
                         const float x = w * 127.0f;
-                        const float ph = __builtin_rintf(x);
-                        const float pl = __builtin_rintf((x - ph) * 127.0f);
-                        pk[row_of(2 * gx + hh, 0) * PROW + key] = (int8_t)(int32_t)ph;
-                        pk[row_of(2 * gx + hh, 1) * PROW + key] = (int8_t)(int32_t)pl;
+                        code[2 * hh] = x + MAGIC;
+                        code[2 * hh + 1] = (x - (code[2 * hh] - MAGIC)) * 127.0f + MAGIC;
                         const float wsum = row16_tree_sum(w);
                         if (nx == 0) (kind ? s.redsum1 : s.redsum)[2 * gx + hh][wave] = wsum;
                     }
+                    *reinterpret_cast<uint32_t *>(pk + key * 16 + 4 * gx) = low_bytes(code[0], code[1], code[2], code[3]);
                 }
                 lds_barrier();
                 // denominator = exp(sink - maximum) + (window tile's pairwise
@@ -1216,8 +1252,7 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
                     const lds_i8 *vbase = (const lds_i8 *)(s.tile[kind]);
 #pragma unroll
                     for (int kb = 0; kb < 2; ++kb) {
-                        const v4i pa = kind ? *reinterpret_cast<const v4i *>(p1 + nx * PROW + 64 * kb + 16 * gx)
-                                            : *reinterpret_cast<const v4i *>(s.p + nx * PROW + 64 * kb + 16 * gx);
+                        const v4i pa = kind ? codes_of((const lds_i8 *)(s.addr), kb, gx, nx) : codes_of((const lds_i8 *)(s.p), kb, gx, nx);
                         const int sl_lo = slot_of(64 * kb + 16 * gx + (nx >> 1));
                         const int sl_hi = slot_of(64 * kb + 16 * gx + 8 + (nx >> 1));
                         v2i b0[4], b1[4];
@@ -1264,19 +1299,27 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
                 const int key = 16 * wave + nx;   // this lane's key in QK and softmax
 
                 // ---- QK: S[16 rows][16 keys of this wave] (reference.py:286-289) ----
+                // Two accumulator chains: half the MFMA latency in a row.
                 v4i sacc = {0, 0, 0, 0};
                 {
                     const int sl = slot_of(key);
-                    v4i b[8];
+                    v4i b[8], other = {0, 0, 0, 0};
 #pragma unroll
                     for (int j = 0; j < 8; ++j) b[j] = *reinterpret_cast<const v4i *>(tb + tile_offset(sl, 4 * j + gx));
                     if (kind) {
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) sacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa1[j], b[j], sacc, 0, 0, 0);
+                        for (int j = 0; j < 8; j += 2) {
+                            sacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa1[j], b[j], sacc, 0, 0, 0);
+                            other = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa1[j + 1], b[j + 1], other, 0, 0, 0);
+                        }
                     } else {
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) sacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa0[j], b[j], sacc, 0, 0, 0);
+                        for (int j = 0; j < 8; j += 2) {
+                            sacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa0[j], b[j], sacc, 0, 0, 0);
+                            other = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa0[j + 1], b[j + 1], other, 0, 0, 0);
+                        }
                     }
+                    sacc += other;
                 }
                 if (stream_next) issue_rows(i + 1, buf ^ 1, DMA_STEP, DMA_STEP);
                 if (held) epilogue();            // the previous tile's, behind this tile's QK
@@ -1291,7 +1334,7 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
                 for (int hh = 0; hh < 2; ++hh) {
                     const int32_t hi = sacc[2 * hh], lo = sacc[2 * hh + 1];
                     float dots = (float)hi;
-                    dots = dots + (float)lo * (float)(1.0 / 127.0);
+                    if (resid) dots = dots + (float)lo * (float)(1.0 / 127.0);
                     const float l = dots * asc[hh];
                     lg[hh] = valid ? l : -1e30f;
                     if (DEBUG && dbg.scores && start + key < klen) {
@@ -1325,22 +1368,22 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
                     factor[1] = odd ? mine : other;
                 }
                 // ---- weights, pairwise tile sum, P codes (reference.py:304-312) ----
+                float code[4];
 #pragma unroll
                 for (int hh = 0; hh < 2; ++hh) {
                     const float w = sk_expf_nonpos(lg[hh] - mnew[hh]);
                     const float x = w * 127.0f;
-                    const float ph = __builtin_rintf(x);
-                    const float pl = resid ? __builtin_rintf((x - ph) * 127.0f) : 0.0f;
-                    s.p[row_of(2 * gx + hh, 0) * PROW + key] = (int8_t)(int32_t)ph;
-                    s.p[row_of(2 * gx + hh, 1) * PROW + key] = (int8_t)(int32_t)pl;
+                    code[2 * hh] = x + MAGIC;
+                    code[2 * hh + 1] = resid ? (x - (code[2 * hh] - MAGIC)) * 127.0f + MAGIC : 0.0f;
                     if (DEBUG && dbg.probs && start + key < klen) {
                         int8_t *drow = reinterpret_cast<int8_t *>(dbg.probs) + ((int64_t)t * positions + (kind ? 128 : 0) + start + key) * 16;
-                        drow[2 * gx + hh] = (int8_t)(int32_t)ph;
-                        drow[8 + 2 * gx + hh] = (int8_t)(int32_t)pl;
+                        drow[2 * gx + hh] = (int8_t)__float_as_int(code[2 * hh]);
+                        drow[8 + 2 * gx + hh] = (int8_t)__float_as_int(code[2 * hh + 1]);
                     }
                     const float wsum = row16_tree_sum(w);   // this wave's 16 keys
                     if (nx == 0) s.redsum[2 * gx + hh][wave] = wsum;
                 }
+                *reinterpret_cast<uint32_t *>(s.p + key * 16 + 4 * gx) = low_bytes(code[0], code[1], code[2], code[3]);
                 lds_barrier();
                 if (stream_next) issue_rows(i + 1, buf ^ 1, 3 * DMA_STEP, DMA_STEP);
 #pragma unroll
@@ -1363,7 +1406,7 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
                     // A: P row nx, keys 64 kb + 16 gx .. + 15.  B: two transposed
                     // 8-key reads; lanes 2r / 2r+1 address the two 8-column halves
                     // of key row r, lane nx receives column nx of the 16-column block.
-                    const v4i pa = *reinterpret_cast<const v4i *>(s.p + nx * PROW + 64 * kb + 16 * gx);
+                    const v4i pa = codes_of((const lds_i8 *)(s.p), kb, gx, nx);
                     const int sl_lo = slot_of(64 * kb + 16 * gx + (nx >> 1));
                     const int sl_hi = slot_of(64 * kb + 16 * gx + 8 + (nx >> 1));
                     v2i b0[4], b1[4];
@@ -1414,8 +1457,10 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
             for (int hh = 0; hh < 2; ++hh) {
                 const int h = 2 * g + hh;
                 if (ANYH && h >= hlive) continue;
+                const float r = 1.0f / den[hh];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) out_row[h * D + c0 + 16 * j + n] = (uint16_t)pack_bf16(num[hh][j] / den[hh], 0.0f);
+                for (int j = 0; j < 4; ++j)
+                    out_row[h * D + c0 + 16 * j + n] = (uint16_t)pack_bf16(div_by(num[hh][j], den[hh], r), 0.0f);
                 if (lse_row && wave == 0 && n == 0) lse_row[h] = mx[hh] + logf(den[hh]);
             }
             if (S > 1 && !fused && tid == 0)
@@ -1482,7 +1527,7 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
     }
 }
 
-template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT>
+template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT, bool RESID>
 __global__ void __launch_bounds__(THREADS, 1)   // one work-group per CU: the 128 KiB tile ring fills the LDS
 c8_attention(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint64_t cmp_indices,
              const uint32_t batch_arg, const uint32_t topk_arg, const uint32_t heads_arg, const uint32_t splits,
@@ -1490,7 +1535,7 @@ c8_attention(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base
              const uint32_t fused)
 {
     __shared__ Shared s;
-    attention_item<RATIO, DEBUG, SLOTS, ANYH, STREAM, JOINT>(s, cu_q, seq_lens, q_base, cmp_indices, batch_arg, topk_arg,
+    attention_item<RATIO, DEBUG, SLOTS, ANYH, STREAM, JOINT, RESID>(s, cu_q, seq_lens, q_base, cmp_indices, batch_arg, topk_arg,
                                                              heads_arg, splits, rows_arg, grid, p, dbg, fused,
                                                              rows_arg * splits);
 }
@@ -1513,30 +1558,6 @@ c8_merge(const SharedKVArgs p, uint32_t splits)
     float *lse_row = p.lse ? reinterpret_cast<float *>(p.lse) + (int64_t)t * H + hbase : nullptr;
     fold_row<0>(row_states(row_partial), folded, threadIdx.x, out_row, lse_row,
                 H - hbase < HEADS ? H - hbase : HEADS);
-}
-
-typedef __attribute__((address_space(3))) v4i lds_v4i;
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-// x rounded to the nearest even integer sits in the low bits of x + MAGIC
-// (|x| < 2^22), so the low byte of the sum is the INT8 code.
-constexpr float MAGIC = 12582912.0f;
-__device__ __forceinline__ uint32_t low_bytes(float a, float b, float c, float d)
-{
-    const uint32_t ab = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x0c0c0400u);
-    const uint32_t cd = __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(c), 0x04000c0cu);
-    return ab | cd;
-}
-
-// num / den, correctly rounded, from the correctly rounded reciprocal r of
-// den: the FMA residual of the product corrects it (Markstein, 1990; den is
-// a softmax denominator, so no operand is subnormal).
-__device__ __forceinline__ float div_by(float num, float den, float r)
-{
-    const float q = num * r;
-    // An infinite quotient's residual is NaN; the median turns that into a
-    // finite number, which leaves the infinity as it is.
-    const float e = __builtin_amdgcn_fmed3f(__builtin_fmaf(-q, den, num), -3.0e38f, 3.0e38f);
-    return __builtin_fmaf(e, r, q);
 }
 
 // ---- launch metadata by wave ballots ----
@@ -2996,7 +3017,7 @@ __device__ __forceinline__ void dma16_at(uint64_t base, uint32_t offset, uint32_
 }
 #pragma clang diagnostic pop
 
-template <int RATIO, bool ANYH>
+template <int RATIO, bool ANYH, bool RESID>
 __global__ void __launch_bounds__(THREADS, 1)
 c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint32_t batch_arg,
          const uint32_t rows_arg, const uint32_t grid, const uint32_t heads_arg, const SharedKVArgs p,
@@ -3015,7 +3036,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
     const int batch_n = (int)batch_arg;
     const int H = ANYH ? (int)heads_arg : HEADS;                 // heads of a query token
     const int HG = ANYH ? (H + HEADS - 1) / HEADS : 1;           // groups of eight
-    const bool resid = !ANYH || H <= HEADS;
+    constexpr bool resid = RESID;
     const int rows_cap = (int)rows_arg;
     // Every wave holds the metadata of the first 64 requests, request b in
     // lane b, and searches them with ballots.
@@ -3083,7 +3104,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
             const int longest = longest_live(cu, lens, live_batch);
             const int live_rows = live_tokens * HG, tiles = 1 + (longest / RATIO + N - 1) / N;
             if (tiles > 1 && PLAN_CUS / live_rows > 1 && !(resid && longest / RATIO <= N)) {
-                attention_item<RATIO, false, false, ANYH, false, true>(
+                attention_item<RATIO, false, false, ANYH, false, RESID, RESID>(
                     *reinterpret_cast<Shared *>(lds), cu_q, seq_lens, q_base, 0, batch_arg, 0, heads_arg, 1, rows_arg, grid,
                     p, SharedKVDebug{0, 0, 0, 0, 0, 0, 0}, fused, rows_arg < grid ? rows_arg : grid);
                 return;
@@ -3370,7 +3391,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
 #pragma unroll
                             for (int hh = 0; hh < 2; ++hh) {
                                 float dots = (float)acc[i][2 * hh];
-                                dots = dots + (float)acc[i][2 * hh + 1] * (float)(1.0 / 127.0);
+                                if (resid) dots = dots + (float)acc[i][2 * hh + 1] * (float)(1.0 / 127.0);
                                 float l = dots * asc[hh];
                                 asm volatile("" : "+v"(l));   // a select, not a branch
                                 lg[b][hh] = valid ? l : -1e30f;
@@ -3478,7 +3499,7 @@ constexpr int PC = 2;
                 }
                 pv(tb, shift, kind, [&](int hh, int c, int hi, int lo, float scale) {
                     float dots = (float)hi;
-                    dots = dots + (float)lo * (float)(1.0 / 127.0);
+                    if (resid) dots = dots + (float)lo * (float)(1.0 / 127.0);
                     num[hh][c] = (kind ? num[hh][c] : 0.0f) * factor[hh] + dots * scale * (float)(1.0 / 127.0);
                 });
             };
@@ -3507,13 +3528,13 @@ constexpr int PC = 2;
                 put_codes(l0);
                 pv(buf, shift, 0, [&](int hh, int c, int hi, int lo, float scale) {
                     float dots = (float)hi;
-                    dots = dots + (float)lo * (float)(1.0 / 127.0);
+                    if (resid) dots = dots + (float)lo * (float)(1.0 / 127.0);
                     num[hh][c] = 0.0f + dots * (scale * (float)(1.0 / 127.0));   // the output starts at 0
                 });
                 put_codes(l1);
                 pv(buf + CHUNK_UNION * D, 0, 1, [&](int hh, int c, int hi, int lo, float scale) {
                     float dots = (float)hi;
-                    dots = dots + (float)lo * (float)(1.0 / 127.0);
+                    if (resid) dots = dots + (float)lo * (float)(1.0 / 127.0);
                     num[hh][c] = num[hh][c] + dots * (scale * (float)(1.0 / 127.0));
                 });
             };
@@ -3798,7 +3819,7 @@ bool xcd_local_dispatch(hipStream_t stream, bool may_probe)
 // them are), which the launch only knows on average.
 constexpr uint32_t CHUNK_MIN_WINDOW = 1024, CHUNK_MIN_C128 = 768, CHUNK_REQUEST_TOKENS = 16;
 
-template <bool DEBUG, bool ANYH>
+template <bool DEBUG, bool ANYH, bool RESID>
 void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDebug &dbg, bool slots, uint32_t grid,
                     uint32_t splits, uint32_t rows, uint32_t fused, bool small_entry)
 {
@@ -3821,7 +3842,7 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
         rows > (a->ratio == 1 ? CHUNK_MIN_WINDOW : CHUNK_MIN_C128) &&
         (uint64_t)a->tokens >= (uint64_t)CHUNK_REQUEST_TOKENS * a->batch) {
         const uint32_t cus = (uint32_t)PLAN_CUS;
-        hipLaunchKernelGGL((a->ratio == 1 ? &c8_chunk<1, ANYH> : &c8_chunk<128, ANYH>), dim3(cus), dim3(THREADS), 0, stream,
+        hipLaunchKernelGGL((a->ratio == 1 ? &c8_chunk<1, ANYH, RESID> : &c8_chunk<128, ANYH, RESID>), dim3(cus), dim3(THREADS), 0, stream,
                            a->cuQ, a->seqLens, a->q, a->batch, rows, cus, a->heads, *a, fused);
         return;
     }
@@ -3840,37 +3861,32 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
         // (Launches of at most PLAN_CUS rows of eight heads stay on
         // c8_attention: 256 rows, 32 sequences of 64 heads, take 23 us there,
         // their 128 wide rows 32 us here.)
-        const uint32_t wide = ANYH && a->heads > HEADS;
+        constexpr bool wide = !RESID;
         const uint32_t own = wide ? a->tokens * ((a->heads + WIDE_HEADS - 1) / WIDE_HEADS) : rows;
         const uint32_t g2 = own < 2u * (uint32_t)PLAN_CUS ? (own + 7u) & ~7u : 2u * (uint32_t)PLAN_CUS;
-        auto rows_kernel = a->ratio == 1 ? &c8_rows<1, false, ANYH, false>
-                           : streamed    ? &c8_rows<4, true, ANYH, false>
-                                         : &c8_rows<4, false, ANYH, false>;
-        if constexpr (ANYH)
-            if (wide)
-                rows_kernel = a->ratio == 1 ? &c8_rows<1, false, true, true>
-                              : streamed    ? &c8_rows<4, true, true, true>
-                                            : &c8_rows<4, false, true, true>;
+        const auto rows_kernel = a->ratio == 1 ? &c8_rows<1, false, ANYH, wide>
+                                 : streamed    ? &c8_rows<4, true, ANYH, wide>
+                                               : &c8_rows<4, false, ANYH, wide>;
         hipLaunchKernelGGL(rows_kernel, dim3(g2), dim3(ROWS_THREADS), 0, stream, a->cuQ, a->seqLens, a->q, a->indices,
                            a->batch, a->topk, rows, g2, a->heads, *a, fused);
         return;
     }
-    decltype(&c8_attention<1, false, false, ANYH, false, false>) kernel =
-        slots ? &c8_attention<1, DEBUG, true, ANYH, false, false>
-              : &c8_attention<1, DEBUG, false, ANYH, false, false>;
+    decltype(&c8_attention<1, false, false, ANYH, false, false, RESID>) kernel =
+        slots ? &c8_attention<1, DEBUG, true, ANYH, false, false, RESID>
+              : &c8_attention<1, DEBUG, false, ANYH, false, false, RESID>;
     if (a->ratio == 4 && joint4)
-        kernel = streamed ? &c8_attention<4, DEBUG, false, ANYH, !DEBUG, !DEBUG>
-                          : &c8_attention<4, DEBUG, false, ANYH, false, !DEBUG>;
+        kernel = streamed ? &c8_attention<4, DEBUG, false, ANYH, !DEBUG, !DEBUG && RESID, RESID>
+                          : &c8_attention<4, DEBUG, false, ANYH, false, !DEBUG && RESID, RESID>;
     else if (a->ratio == 4)
-        kernel = slots ? (streamed ? &c8_attention<4, DEBUG, true, ANYH, !DEBUG, false>
-                                   : &c8_attention<4, DEBUG, true, ANYH, false, false>)
-                       : (streamed ? &c8_attention<4, DEBUG, false, ANYH, !DEBUG, false>
-                                   : &c8_attention<4, DEBUG, false, ANYH, false, false>);
+        kernel = slots ? (streamed ? &c8_attention<4, DEBUG, true, ANYH, !DEBUG, false, RESID>
+                                   : &c8_attention<4, DEBUG, true, ANYH, false, false, RESID>)
+                       : (streamed ? &c8_attention<4, DEBUG, false, ANYH, !DEBUG, false, RESID>
+                                   : &c8_attention<4, DEBUG, false, ANYH, false, false, RESID>);
     else if (a->ratio == 128)
-        kernel = slots ? (streamed ? &c8_attention<128, DEBUG, true, ANYH, !DEBUG, true>
-                                   : &c8_attention<128, DEBUG, true, ANYH, false, true>)
-                       : (streamed ? &c8_attention<128, DEBUG, false, ANYH, !DEBUG, true>
-                                   : &c8_attention<128, DEBUG, false, ANYH, false, true>);
+        kernel = slots ? (streamed ? &c8_attention<128, DEBUG, true, ANYH, !DEBUG, RESID, RESID>
+                                   : &c8_attention<128, DEBUG, true, ANYH, false, RESID, RESID>)
+                       : (streamed ? &c8_attention<128, DEBUG, false, ANYH, !DEBUG, RESID, RESID>
+                                   : &c8_attention<128, DEBUG, false, ANYH, false, RESID, RESID>);
     // The leading scalar arguments are the ones the first loads need; the
     // build preloads them into SGPRs (-amdgpu-kernarg-preload-count), so
     // those loads do not wait for a read of the argument block.
@@ -3906,10 +3922,13 @@ int launch_attention(hipStream_t stream, const SharedKVArgs *a, const SharedKVDe
     // Debug dumps hold eight heads and one original tile (list places 0..127) per row.
     if (DEBUG && (a->heads != HEADS || (a->oriIndices && a->oriTopk > N))) return (int)hipErrorInvalidValue;
     const bool slots = a->oriIndices != 0;
-    if (!DEBUG && a->heads != HEADS)
-        launch_variant<false, true>(stream, a, dbg, slots, grid, splits, rows, fused, small_entry);
+    // Above eight heads no residual codes (reference.py:221-222).
+    if (!DEBUG && a->heads > HEADS)
+        launch_variant<false, true, false>(stream, a, dbg, slots, grid, splits, rows, fused, small_entry);
+    else if (!DEBUG && a->heads != HEADS)
+        launch_variant<false, true, true>(stream, a, dbg, slots, grid, splits, rows, fused, small_entry);
     else
-        launch_variant<DEBUG, false>(stream, a, dbg, slots, grid, splits, rows, fused, small_entry);
+        launch_variant<DEBUG, false, true>(stream, a, dbg, slots, grid, splits, rows, fused, small_entry);
     if (splits > 1 && !fused)
         hipLaunchKernelGGL(c8_merge, dim3(rows), dim3(THREADS), 0, stream, *a, splits);
     return (int)hipGetLastError();
