@@ -3386,19 +3386,24 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
 #pragma unroll
                         for (int i = 0; i < 2; ++i) {
                             const int b = st - 1 + i;
-                            const int most = (pages >> (b >> 1)) & 1u ? live : 0;
-                            const bool valid = nx < most - 16 * b;
 #pragma unroll
                             for (int hh = 0; hh < 2; ++hh) {
                                 float dots = (float)acc[i][2 * hh];
                                 if (resid) dots = dots + (float)acc[i][2 * hh + 1] * (float)(1.0 / 127.0);
-                                float l = dots * asc[hh];
-                                asm volatile("" : "+v"(l));   // a select, not a branch
-                                lg[b][hh] = valid ? l : -1e30f;
+                                lg[b][hh] = dots * asc[hh];
                             }
                         }
                     }
                     __builtin_amdgcn_sched_barrier(0);
+                }
+                if (live < N || pages != 15u) {   // some of the tile's keys are not the row's
+#pragma unroll
+                    for (int b = 0; b < 8; ++b) {
+                        const int most = (pages >> (b >> 1)) & 1u ? live : 0;
+                        const bool valid = nx < most - 16 * b;
+#pragma unroll
+                        for (int hh = 0; hh < 2; ++hh) lg[b][hh] = valid ? lg[b][hh] : -1e30f;
+                    }
                 }
                 if (in_window && __ballot(s.bad[which][lane & (CHUNK_ROWS - 1)])) {
 #pragma unroll
