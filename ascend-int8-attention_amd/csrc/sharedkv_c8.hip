@@ -1641,7 +1641,7 @@ __device__ __forceinline__ Request find_request(global_i32 cu, global_i32 lens, 
 // memory.  Each wave takes 32 keys in QK (the rows it copied: no barrier
 // before it) and 128 output columns in PV.
 // Bound by instruction issue: 391 VALU instructions a wave and tile (most of
-// them the FP32 sequence), VALU 62 % and LDS 40 % busy; with every row an L2
+// them the FP32 sequence), VALU 58 % and LDS 42 % busy; with every row an L2
 // hit a prefill chunk takes the same time.  Eight waves a work-group at 128
 // VGPRs were slower (130 against 116 us on the chunk below).
 // Measured on MI355X, LDS DMA copies and rows of eight heads -> this: decode
@@ -2990,10 +2990,10 @@ c8_pairs(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
 // Bound by the FP32 sequence (about 1250 VALU instructions a wave and tile,
 // 4.2 us for the two waves of a SIMD) and the LDS reads (1 MiB a tile and
 // work-group, 3.4 us), which overlap only in part: a tile takes about 6 us, a
-// window-only octet about 15.  Measured on MI355X, before -> after: B = 1 x
-// T = 2048, C128 at 8 K / 32 K / 128 K context 62 / 79 / 160 -> 27 / 33 / 69
-// us, window-only 26 -> 17; T = 4096 C128 at 32 K 156 -> 62, window-only
-// 48 -> 32.
+// window-only octet about 15.  Three requests of 662 C128 rows: VALU 72 %, LDS
+// 24 % busy.  Measured on MI355X, before -> after: B = 1 x T = 2048, C128 at
+// 8 K / 32 K / 128 K context 62 / 79 / 160 -> 27 / 33 / 68 us, window-only
+// 26 -> 17.5; T = 4096 C128 at 32 K 156 -> 62, window-only 48 -> 31.
 constexpr int CHUNK_ROWS = 8;                        // query rows of a work-group (one per wave)
 constexpr int CHUNK_UNION = N + CHUNK_ROWS;          // window rows of an octet (135 at most), in pairs
 constexpr int OUT_STRIDE = 2 * D + 32;               // LDS row stride of a head's BF16 output
@@ -3814,15 +3814,33 @@ bool xcd_local_dispatch(hipStream_t stream, bool may_probe)
     return ok;
 }
 
-// Launches of c8_chunk: a work-group takes eight rows in about the time of one
-// (window-only 15 us, C128 at 8 K / 32 K context 24 / 30 us for any row count
-// up to 2048), so they need enough rows.  Window-only: 1024 rows take 16.1 us
-// on c8_chunk and 14.4 on c8_rows, 1500 rows 16.5 and 20.2.  C128: 700 rows
-// 24.6 and 24.3 at 8 K (30.8 and 30.7 at 32 K) against c8_attention, 1024 rows
-// 24.8 and 31.9 (30.8 and 40.6).  And the rows of a work-group have to come
-// from few requests (1024 rows of 128 requests are no slower, 512 rows of
-// them are), which the launch only knows on average.
-constexpr uint32_t CHUNK_MIN_WINDOW = 1024, CHUNK_MIN_C128 = 768, CHUNK_REQUEST_TOKENS = 16;
+// Launches of c8_chunk: a work-group takes eight rows in about the time of one,
+// so that up to 2048 rows of eight heads cost about the same (window-only
+// 17 us, C128 at 8 K / 32 K context 27 / 33 us).
+// Window-only, against c8_rows: a round of 2048 rows takes about as long as
+// three rounds of its 512 rows (1024 rows 13.0 us on c8_rows and 17.0 on
+// c8_chunk, 1150 rows 17.3 and 17.0, 2048 21.8 and 17.7, 2100-2560 26.3 and
+// 29.9, 3000 30.9 and 30.1, 4096 40.2 and 31.4, 8192 77 and 59), or as two
+// rounds of 512 rows of sixteen heads above eight heads (16 heads, T = 512
+// 9.8 and 15.4, 600 17.5 and 15.6, 1024 18.1 and 16.5, 1500 24.1 and 27.1,
+// 2048 30.6 and 27.9; 64 heads, T = 2048 108 and 98).
+// C128, against c8_attention's rounds of 256 rows: 768 rows 23.6 and 26.8 us
+// at 8 K (30.0 and 32.8 at 32 K), 1024 rows 30.6 and 26.9 (39.4 and 32.7).
+// And the rows of a work-group have to come from few requests (1024 rows of
+// 128 requests are no slower, 512 rows of them are), which the launch only
+// knows on average.
+constexpr uint32_t CHUNK_ROUND = CHUNK_ROWS * PLAN_CUS, ROWS_ROUND = 2 * PLAN_CUS;
+constexpr uint32_t CHUNK_MIN_C128 = 768, CHUNK_REQUEST_TOKENS = 16;
+
+// `own`: the launch's rows as c8_rows counts them.
+template <bool WIDE>
+bool chunk_launch(const SharedKVArgs *a, uint32_t rows, uint32_t own)
+{
+    if ((uint64_t)a->tokens < (uint64_t)CHUNK_REQUEST_TOKENS * a->batch) return false;
+    if (a->ratio == 128) return rows > CHUNK_MIN_C128;
+    const uint64_t rounds = ((uint64_t)rows + CHUNK_ROUND - 1) / CHUNK_ROUND;
+    return a->ratio == 1 && rounds * (WIDE ? 2 : 3) <= ((uint64_t)own + ROWS_ROUND - 1) / ROWS_ROUND;
+}
 
 template <bool DEBUG, bool ANYH, bool RESID>
 void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDebug &dbg, bool slots, uint32_t grid,
@@ -3843,9 +3861,9 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
                         (small_entry || (uint64_t)a->cmpTableWidth * BLOCK_ROWS <= (uint64_t)N);
     // Prefill-shaped C128 and window-only launches share KV tiles between
     // neighbouring rows.
-    if (!DEBUG && !slots && splits == 1 && a->ratio != 4 &&
-        rows > (a->ratio == 1 ? CHUNK_MIN_WINDOW : CHUNK_MIN_C128) &&
-        (uint64_t)a->tokens >= (uint64_t)CHUNK_REQUEST_TOKENS * a->batch) {
+    constexpr bool wide = !RESID;
+    const uint32_t own = wide ? a->tokens * ((a->heads + WIDE_HEADS - 1) / WIDE_HEADS) : rows;
+    if (!DEBUG && !slots && splits == 1 && chunk_launch<wide>(a, rows, own)) {
         const uint32_t cus = (uint32_t)PLAN_CUS;
         hipLaunchKernelGGL((a->ratio == 1 ? &c8_chunk<1, ANYH, RESID> : &c8_chunk<128, ANYH, RESID>), dim3(cus), dim3(THREADS), 0, stream,
                            a->cuQ, a->seqLens, a->q, a->batch, rows, cus, a->heads, *a, fused);
@@ -3854,9 +3872,9 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
     // One-partition C4 and window-only launches of more rows than CUs
     // (prefill, large decode batches) without explicit slots run two
     // four-wave work-groups per CU taking rows in turn (c8_rows; above eight
-    // heads rows of sixteen).  Other C128
-    // launches keep one work-group per row: c8_attention's two-tile ring
-    // measured faster on them (decode of 512 rows 51 against 72 us).
+    // heads rows of sixteen).  Other C128 launches keep one work-group per
+    // row: c8_attention's two-tile ring measured faster on them (decode of 512
+    // rows 51 against 72 us).
     const bool persist = !DEBUG && !slots && splits == 1 && rows > (uint32_t)PLAN_CUS &&
                          (a->ratio == 1 || (a->ratio == 4 && !joint4));
     if (persist) {
@@ -3866,8 +3884,6 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
         // (Launches of at most PLAN_CUS rows of eight heads stay on
         // c8_attention: 256 rows, 32 sequences of 64 heads, take 23 us there,
         // their 128 wide rows 32 us here.)
-        constexpr bool wide = !RESID;
-        const uint32_t own = wide ? a->tokens * ((a->heads + WIDE_HEADS - 1) / WIDE_HEADS) : rows;
         const uint32_t g2 = own < 2u * (uint32_t)PLAN_CUS ? (own + 7u) & ~7u : 2u * (uint32_t)PLAN_CUS;
         const auto rows_kernel = a->ratio == 1 ? &c8_rows<1, false, ANYH, wide>
                                  : streamed    ? &c8_rows<4, true, ANYH, wide>

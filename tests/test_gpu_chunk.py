@@ -1,8 +1,8 @@
 """Prefill-shaped C128 and window-only launches (c8_chunk: one query row per
 wave, eight neighbouring rows of a work-group sharing their KV tiles): how the
 octets of rows meet requests, padding, joint rows, head groups and unreadable
-pages.  Bit-exact with the checker on the launch's plan; every launch here is
-large enough for that kernel (more than 1024 window-only rows or 768 C128 rows,
+pages.  Bit-exact with the oracle on the launch's plan; every launch here is
+one that kernel takes (1025-2048 window-only rows or more than 768 C128 rows,
 16 query tokens per request on average)."""
 import sys
 
@@ -51,13 +51,13 @@ CASES = [
 
 
 @pytest.mark.parametrize("name,ratio,queries,lengths,heads,pad", CASES, ids=[c[0] for c in CASES])
-def test_chunk_launch_matches_checker(name, ratio, queries, lengths, heads, pad):
+def test_chunk_launch_matches_oracle(name, ratio, queries, lengths, heads, pad):
     from npu_sparse_attn_sharedkv_int8 import c8_attention
     say(f"[chunk] {name}")
     case = workloads.make_case(90, ratio, queries, lengths, heads=heads)
     launch = padded(case, pad) if pad else case
     rows = launch["q"].shape[0] * ((heads + 7) // 8)
-    assert rows > (1024 if ratio == 1 else 768) and launch["q"].shape[0] >= 16 * len(launch["seq_lens"])
+    assert (1024 < rows <= 2048 if ratio == 1 else rows > 768) and launch["q"].shape[0] >= 16 * len(launch["seq_lens"])
     out, lse, op = run_hip(launch, splits=1)
     plan, joint = op.device_splits(), joint_flags(launch, 1)
     assert (plan > 1) == (name == "replanned")
@@ -66,7 +66,7 @@ def test_chunk_launch_matches_checker(name, ratio, queries, lengths, heads, pad)
     dead = c8_attention.keyless_tokens(case["cu_q"], case["seq_lens"], live)
     keep = [t for t in range(live) if not dead[t]]
     assert not out[[t for t in range(live) if dead[t]]].any(), "keyless rows are not zero"
-    # The launch's own requests where the checker takes them, else one request per row.
+    # The launch's own requests where the oracle takes them, else one request per row.
     sub = case if len(keep) == live else query_subcase(case, keep)
     ref, ref_lse, _ = run_oracle(sub, plan, joint=joint)
     diff = out[keep] != ref

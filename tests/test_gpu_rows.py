@@ -2,7 +2,7 @@
 heads, above eight heads): head counts that leave a row or a group of eight
 part full, both load policies, masked entries, and padded launches re-planned
 into partitions, whose states and tickets count rows of eight heads.  Bit-exact
-with the checker on the launch's plan."""
+with the oracle on the launch's plan."""
 import sys
 
 import numpy as np
@@ -27,7 +27,7 @@ CASES = [
 
 
 @pytest.mark.parametrize("name,ratio,queries,lengths,heads,mode,pad", CASES, ids=[c[0] for c in CASES])
-def test_wide_rows_match_checker(name, ratio, queries, lengths, heads, mode, pad):
+def test_wide_rows_match_oracle(name, ratio, queries, lengths, heads, mode, pad):
     print(f"[wide rows] {name}", file=sys.stderr, flush=True)
     case = workloads.make_case(92, ratio, queries, lengths, heads=heads, index_mode=mode)
     launch = case
