@@ -202,8 +202,10 @@ def device_splits(splits, tokens, heads, ratio, topk, cu_q, seq_lens, ori_topk=0
 
 
 def rows_launch(splits, tokens, heads, ratio, ori_topk=0, cmp_rows=None, small=None):
-    """Whether the kernel runs a launch on c8_rows (two four-wave work-groups
-    per CU taking rows in turn): one partition, more rows than CUs, no
+    """Whether a launch's rows are its work-groups in the kernel's re-plan, as
+    on c8_rows (two four-wave work-groups per CU taking rows in turn; large
+    window-only launches run c8_chunk, where one tile is one partition either
+    way): one partition, more rows than CUs, no
     explicit original slots, and window-only or C4 without joint rows
     compiled in (C4 kernels carry them for launches through the small-launch
     entry and for compressed block tables of at most one tile of rows per
