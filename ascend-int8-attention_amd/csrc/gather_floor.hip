@@ -31,16 +31,18 @@ struct alignas(16) FloorShared {
 };
 
 // LDS DMA of 16 bytes per lane (lane l's bytes land at lds + 16 l); M0
-// carries the LDS address.
+// carries the LDS address (one wait state after its scalar write).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 template <bool NT>
 __device__ __forceinline__ void dma16(uint64_t src, uint32_t lds)
 {
     if (NT)
-        asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt" :: "v"(src), "s"(lds) : "memory", "m0");
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
+                     :: "v"(src), "s"(lds) : "memory", "m0");
     else
-        asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(src), "s"(lds) : "memory", "m0");
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                     :: "v"(src), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop
 

@@ -245,7 +245,9 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // not track it: its own tracking cannot tell the two ring buffers apart and
 // would wait for the next tile's DMA before every LDS read.  The callers
 // order these copies with vm_wait and lds_barrier instead.  M0 carries the
-// LDS address (the compiler keeps nothing live in M0 in this file).  NT sets
+// LDS address (the compiler keeps nothing live in M0 in this file); the ISA
+// asks for one wait state between a scalar write of M0 and an LDS DMA, which
+// the compiler does not add inside inline assembly.  NT sets
 // the non-temporal cache policy, for launches whose KV rows are read about
 // once (decode: few query tokens per sequence).  Prefill launches, whose
 // query tokens re-read the same rows from L2, keep the default policy.
@@ -255,9 +257,11 @@ template <bool NT>
 __device__ __forceinline__ void dma16(uint64_t src, uint32_t lds)
 {
     if (NT)
-        asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt" :: "v"(src), "s"(lds) : "memory", "m0");
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
+                     :: "v"(src), "s"(lds) : "memory", "m0");
     else
-        asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(src), "s"(lds) : "memory", "m0");
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                     :: "v"(src), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop
 
@@ -3013,7 +3017,8 @@ static_assert(CHUNK_ROWS * HEADS * OUT_STRIDE <= CHUNK_UNION * D, "output stagin
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16_at(uint64_t base, uint32_t offset, uint32_t lds)
 {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(offset), "s"(base), "s"(lds) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(offset), "s"(base), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop
 

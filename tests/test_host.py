@@ -414,3 +414,16 @@ def test_case_to_moves_every_tensor():
     case = cpu_case()
     moved = case.to("cpu")
     assert moved is not case and moved.ratio == 4 and torch.equal(moved.q, case.q)
+
+
+def test_lds_dma_waits_after_its_m0_write():
+    """gfx9 asks for a wait state between a scalar write of M0 and an LDS DMA
+    load that uses it (the compiler puts an s_nop there for its own builtin);
+    inline assembly has to hold it itself."""
+    seen = 0
+    for source in (ROOT / "ascend-int8-attention_amd" / "csrc").glob("*.hip"):
+        for block in re.findall(r'asm volatile\(\s*"([^"]*_load_lds_[^"]*)"', source.read_text()):
+            seen += 1
+            steps = [step.split()[0] for step in block.split(r"\n\t")]
+            assert steps[0] == "s_mov_b32" and steps[1] == "s_nop" and len(steps) == 3, f"{source.name}: {block}"
+    assert seen == 5
