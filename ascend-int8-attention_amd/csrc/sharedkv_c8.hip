@@ -510,27 +510,31 @@ __device__ __forceinline__ void fold_row(const __amdgpu_buffer_rsrc_t states, in
 // written.  Above eight heads the Q and P residual codes are zero
 // (reference.py:221-222: residual quantization only for <= 8 heads), which
 // leaves every other operation as it is.  Without ANYH, heads == 8.
-// The work of one work-group: item `item` of the launch's `items`.
-template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT, bool RESID>
+// The work of one work-group: work-group `block` of a launch of `grid` (a
+// multiple of 8) with `items` work items.
+// TIGHT: nothing derived from the thread is held in a register from before
+// the row codes on (inside c8_chunk, whose scalar spills take registers).
+template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT, bool RESID, bool TIGHT>
 __device__ __forceinline__ void
 attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint64_t cmp_indices,
                const uint32_t batch_arg, const uint32_t topk_arg, const uint32_t heads_arg, const uint32_t splits,
                const uint32_t rows_arg, const uint32_t grid, const SharedKVArgs &p, const SharedKVDebug &dbg,
-               const uint32_t fused, const uint32_t items)
+               const uint32_t fused, const uint32_t items, const uint32_t block, int tid)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
+    int lane = tid & 63, wave = tid >> 6;
+    const int g = lane >> 4, n = lane & 15;
 
     // XCD-aware order: consecutive work items (the partitions of one row,
     // then the next row) stay on one XCD and share its L2: XCD x takes the
     // items [x G / 8, (x + 1) G / 8).
     const uint32_t G = grid;
-    const uint32_t item = (blockIdx.x & 7u) * (G >> 3) + (blockIdx.x >> 3);
+    const uint32_t item = (block & 7u) * (G >> 3) + (block >> 3);
     if (item >= items) return;
     const int H = ANYH ? (int)heads_arg : HEADS;                 // heads of a query token
     const int HG = ANYH ? (H + HEADS - 1) / HEADS : 1;           // groups of eight
     constexpr bool resid = RESID;
     // The launch's plan: `splits` partitions per row over rows_arg rows.
-    // rows.  The work item's row under that plan is loaded at once; with
+    // The work item's row under that plan is loaded at once; with
     // graph padding the device re-plans (below) and may move it.
     int32_t S = (int32_t)splits;
     int32_t qrow = (int32_t)(item / splits);                     // (token, head group)
@@ -687,7 +691,7 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
         int32_t row;
         const int32_t per_xcd = (int32_t)(G >> 3), usable = per_xcd - (int32_t)(G - items);
         if ((live_rows + 7) / 8 * plan <= usable) {
-            const int32_t x = (int32_t)(blockIdx.x & 7u), j = (int32_t)(blockIdx.x >> 3);
+            const int32_t x = (int32_t)(block & 7u), j = (int32_t)(block >> 3);
             row = x * live_rows / 8 + j / plan;
             if (row >= (x + 1) * live_rows / 8) return;
             part = j % plan;
@@ -1011,6 +1015,7 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
         constexpr bool ONE_CHUNK = RATIO == 4 && !SLOTS;
         for (int first = 0; first < my_tiles && (!ONE_CHUNK || first == 0); first += CODE_TILES) {
             const int ntiles = my_tiles - first < CODE_TILES ? my_tiles - first : CODE_TILES;
+            if (TIGHT) asm volatile("" : "+v"(tid), "+v"(lane), "+v"(wave));
             // ---- row codes of partition tiles [first, first + ntiles) ----
             for (int i = tid; i < ntiles * N; i += THREADS) {
                 s.code[i] = -1;
@@ -1539,9 +1544,9 @@ c8_attention(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base
              const uint32_t fused)
 {
     __shared__ Shared s;
-    attention_item<RATIO, DEBUG, SLOTS, ANYH, STREAM, JOINT, RESID>(s, cu_q, seq_lens, q_base, cmp_indices, batch_arg, topk_arg,
+    attention_item<RATIO, DEBUG, SLOTS, ANYH, STREAM, JOINT, RESID, false>(s, cu_q, seq_lens, q_base, cmp_indices, batch_arg, topk_arg,
                                                              heads_arg, splits, rows_arg, grid, p, dbg, fused,
-                                                             rows_arg * splits);
+                                                             rows_arg * splits, blockIdx.x, (int)threadIdx.x);
 }
 
 // Partition merge as a second launch (merge mode 1): one 512-thread group
@@ -3022,6 +3027,37 @@ __device__ __forceinline__ void dma16_at(uint64_t base, uint32_t offset, uint32_
 }
 #pragma clang diagnostic pop
 
+// Launches of c8_chunk: a work-group takes eight rows in about the time of one,
+// so that up to 2048 rows of eight heads cost about the same (window-only
+// 17 us, C128 at 8 K / 32 K context 27 / 33 us).
+// Window-only, against c8_rows: a round of 2048 rows takes about as long as
+// three rounds of its 512 rows (1024 rows 13.0 us on c8_rows and 17.0 on
+// c8_chunk, 1150 rows 17.3 and 17.0, 2048 21.8 and 17.7, 2100-2560 26.3 and
+// 29.9, 3000 30.9 and 30.1, 4096 40.2 and 31.4, 8192 77 and 59), or as two
+// rounds of 512 rows of sixteen heads above eight heads (16 heads, T = 512
+// 9.8 and 15.4, 600 17.5 and 15.6, 1024 18.1 and 16.5, 1500 24.1 and 27.1,
+// 2048 30.6 and 27.9; 64 heads, T = 2048 108 and 98).
+// C128, against c8_attention's rounds of 256 rows: 768 rows 23.6 and 26.8 us
+// at 8 K (30.0 and 32.8 at 32 K), 1024 rows 30.6 and 26.9 (39.4 and 32.7).
+// And the rows of a work-group have to come from few requests (1024 rows of
+// 128 requests are no slower, 512 rows of them are), which the launch only
+// knows on average.
+// The host decides with a launch's own shape; for graph padding the kernel
+// decides again with the live one.
+constexpr uint32_t CHUNK_ROUND = CHUNK_ROWS * PLAN_CUS, ROWS_ROUND = 2 * PLAN_CUS;
+constexpr uint32_t CHUNK_MIN_C128 = 768, CHUNK_REQUEST_TOKENS = 16;
+
+// `rows` rows of eight heads of `tokens` query tokens and `batch` requests
+// take `rounds` rounds of octets; `own`: the rows as c8_rows counts them.
+template <bool WIDE>
+__host__ __device__ constexpr bool chunk_pays(int ratio, uint32_t tokens, uint32_t batch, uint32_t rows, uint32_t own,
+                                              uint32_t rounds)
+{
+    if ((uint64_t)tokens < (uint64_t)CHUNK_REQUEST_TOKENS * batch) return false;
+    if (ratio == 128) return rows > CHUNK_MIN_C128;
+    return ratio == 1 && (uint64_t)rounds * (WIDE ? 2 : 3) <= ((uint64_t)own + ROWS_ROUND - 1) / ROWS_ROUND;
+}
+
 template <int RATIO, bool ANYH, bool RESID>
 __global__ void __launch_bounds__(THREADS, 1)
 c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint32_t batch_arg,
@@ -3101,17 +3137,31 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
             zero_row(ANYH ? row / HG : row, h, ANYH ? (H - h < HEADS ? H - h : HEADS) : HEADS);
         }
         if (live_tokens == 0) return;
-        if (RATIO == 128 && fused) {
+        if (RATIO == 128) {
             // c8_attention's device plan: few live rows run as several
             // partitions each (its rule, c8_attention.device_splits on the
             // host, over this launch's work-groups), unless every row is a
             // joint row.
             const int longest = longest_live(cu, lens, live_batch);
             const int live_rows = live_tokens * HG, tiles = 1 + (longest / RATIO + N - 1) / N;
-            if (tiles > 1 && PLAN_CUS / live_rows > 1 && !(resid && longest / RATIO <= N)) {
-                attention_item<RATIO, false, false, ANYH, false, RESID, RESID>(
-                    *reinterpret_cast<Shared *>(lds), cu_q, seq_lens, q_base, 0, batch_arg, 0, heads_arg, 1, rows_arg, grid,
-                    p, SharedKVDebug{0, 0, 0, 0, 0, 0, 0}, fused, rows_arg < grid ? rows_arg : grid);
+            const bool plan =
+                fused && tiles > 1 && PLAN_CUS / live_rows > 1 && !(resid && longest / RATIO <= N);
+            // Otherwise the launch rule on the live shape: octets or, where an
+            // eager launch of the live rows would not come here,
+            // c8_attention's rows, one work-group each in turn.
+            if (plan || !chunk_pays<!RESID>(RATIO, live_tokens, live_batch, live_rows, live_rows, 0)) {
+                __builtin_amdgcn_s_setprio(0);
+                const uint32_t of_rows = plan ? rows_arg : (uint32_t)live_rows;
+                const uint32_t groups = plan ? grid : ((uint32_t)live_rows + 7u) & ~7u;
+                const uint32_t items = of_rows < groups ? of_rows : groups;
+                for (uint32_t block = blockIdx.x; block < groups; block += grid) {
+                    int thread = (int)threadIdx.x;   // opaque: no per-lane value is held across the rows
+                    asm volatile("" : "+v"(thread));
+                    attention_item<RATIO, false, false, ANYH, false, RESID, RESID, true>(
+                        *reinterpret_cast<Shared *>(lds), cu_q, seq_lens, q_base, 0, batch_arg, 0, heads_arg, 1, of_rows,
+                        groups, p, SharedKVDebug{0, 0, 0, 0, 0, 0, 0}, fused, items, block, thread);
+                    __syncthreads();
+                }
                 return;
             }
         }
@@ -3819,34 +3869,6 @@ bool xcd_local_dispatch(hipStream_t stream, bool may_probe)
     return ok;
 }
 
-// Launches of c8_chunk: a work-group takes eight rows in about the time of one,
-// so that up to 2048 rows of eight heads cost about the same (window-only
-// 17 us, C128 at 8 K / 32 K context 27 / 33 us).
-// Window-only, against c8_rows: a round of 2048 rows takes about as long as
-// three rounds of its 512 rows (1024 rows 13.0 us on c8_rows and 17.0 on
-// c8_chunk, 1150 rows 17.3 and 17.0, 2048 21.8 and 17.7, 2100-2560 26.3 and
-// 29.9, 3000 30.9 and 30.1, 4096 40.2 and 31.4, 8192 77 and 59), or as two
-// rounds of 512 rows of sixteen heads above eight heads (16 heads, T = 512
-// 9.8 and 15.4, 600 17.5 and 15.6, 1024 18.1 and 16.5, 1500 24.1 and 27.1,
-// 2048 30.6 and 27.9; 64 heads, T = 2048 108 and 98).
-// C128, against c8_attention's rounds of 256 rows: 768 rows 23.6 and 26.8 us
-// at 8 K (30.0 and 32.8 at 32 K), 1024 rows 30.6 and 26.9 (39.4 and 32.7).
-// And the rows of a work-group have to come from few requests (1024 rows of
-// 128 requests are no slower, 512 rows of them are), which the launch only
-// knows on average.
-constexpr uint32_t CHUNK_ROUND = CHUNK_ROWS * PLAN_CUS, ROWS_ROUND = 2 * PLAN_CUS;
-constexpr uint32_t CHUNK_MIN_C128 = 768, CHUNK_REQUEST_TOKENS = 16;
-
-// `own`: the launch's rows as c8_rows counts them.
-template <bool WIDE>
-bool chunk_launch(const SharedKVArgs *a, uint32_t rows, uint32_t own)
-{
-    if ((uint64_t)a->tokens < (uint64_t)CHUNK_REQUEST_TOKENS * a->batch) return false;
-    if (a->ratio == 128) return rows > CHUNK_MIN_C128;
-    const uint64_t rounds = ((uint64_t)rows + CHUNK_ROUND - 1) / CHUNK_ROUND;
-    return a->ratio == 1 && rounds * (WIDE ? 2 : 3) <= ((uint64_t)own + ROWS_ROUND - 1) / ROWS_ROUND;
-}
-
 template <bool DEBUG, bool ANYH, bool RESID>
 void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDebug &dbg, bool slots, uint32_t grid,
                     uint32_t splits, uint32_t rows, uint32_t fused, bool small_entry)
@@ -3868,7 +3890,8 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
     // neighbouring rows.
     constexpr bool wide = !RESID;
     const uint32_t own = wide ? a->tokens * ((a->heads + WIDE_HEADS - 1) / WIDE_HEADS) : rows;
-    if (!DEBUG && !slots && splits == 1 && chunk_launch<wide>(a, rows, own)) {
+    const uint32_t rounds = (uint32_t)(((uint64_t)rows + CHUNK_ROUND - 1) / CHUNK_ROUND);
+    if (!DEBUG && !slots && splits == 1 && chunk_pays<wide>((int)a->ratio, a->tokens, a->batch, rows, own, rounds)) {
         const uint32_t cus = (uint32_t)PLAN_CUS;
         hipLaunchKernelGGL((a->ratio == 1 ? &c8_chunk<1, ANYH, RESID> : &c8_chunk<128, ANYH, RESID>), dim3(cus), dim3(THREADS), 0, stream,
                            a->cuQ, a->seqLens, a->q, a->batch, rows, cus, a->heads, *a, fused);

@@ -1,0 +1,83 @@
+"""Prefill launches at a graph's capacity with few live rows: the kernel that
+the capacity selects (c8_chunk) runs them as the kernel that an eager launch of
+the live rows would run, bit-exact with the oracle and in about its time."""
+import sys
+
+import numpy as np
+import pytest
+
+from tests import workloads
+from tests.device_cases import DeviceCase, joint_flags, run_hip, run_oracle
+from tests.test_gpu_chunk import padded
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # name, ratio, queries, lengths, heads, padding rows
+    ("two_passes", 128, [300, 9], [17000, 700], 8, 900),           # 309 rows over 256 work-groups
+    ("most_rows", 128, [768], [16900], 8, 300),                    # the last count that takes whole rows
+    ("octets", 128, [769], [16900], 8, 300),                       # and the first that takes octets
+    ("joint", 128, [290, 40], [3000, 700], 8, 900),                # every row joint, two passes
+    ("head_groups", 128, [150, 40], [17000, 2500], 20, 400),       # 570 rows of three groups
+    ("many_requests", 128, [4] * 210, list(range(300, 300 + 210 * 90, 90)), 8, 2600),   # 840 rows, four a request
+]
+
+
+@pytest.mark.parametrize("name,ratio,queries,lengths,heads,pad", CASES, ids=[c[0] for c in CASES])
+def test_padded_launch_matches_oracle(name, ratio, queries, lengths, heads, pad):
+    print(f"[padded] {name}", file=sys.stderr, flush=True)
+    case = workloads.make_case(93, ratio, queries, lengths, heads=heads)
+    launch = padded(case, pad)
+    rows, live = launch["q"].shape[0] * ((heads + 7) // 8), int(case["cu_q"][-1])
+    assert (rows > 1024 if ratio == 1 else rows > 768) and launch["q"].shape[0] >= 16 * len(launch["seq_lens"])
+    out, lse, op = run_hip(launch, splits=1)
+    assert op.device_splits() == 1
+    assert not out[live:].any() and not lse[live:].any(), "padding rows are not zero"
+    ref, ref_lse, _ = run_oracle(case, 1, joint=joint_flags(launch, 1))
+    diff = out[:live] != ref
+    assert not diff.any(), f"{int(diff.sum())} BF16 mismatches, rows {sorted(set(np.argwhere(diff)[:, 0]))[:8]}"
+    np.testing.assert_allclose(lse[:live], ref_lse, rtol=0, atol=2e-6)
+
+
+def microseconds(call, calls=50, rounds=7):
+    import torch
+    for _ in range(5):
+        call()
+    times = []
+    for _ in range(rounds):
+        first, last = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        first.record()
+        for _ in range(calls):
+            call()
+        last.record()
+        torch.cuda.synchronize()
+        times.append(first.elapsed_time(last) * 1000 / calls)
+    return sorted(times)[rounds // 2]
+
+
+@pytest.mark.parametrize("ratio,live,length", [(128, 40, 6000), (128, 200, 32768), (128, 200, 131072)])
+def test_padded_launch_takes_the_time_of_its_live_rows(ratio, live, length):
+    """A launch of 2048 query tokens with `live` live ones takes no more than
+    1.5 times an eager launch of those and a fill of the padding's outputs
+    together (measured: 0.9-1.2 times; an octet of eight rows on each of a few
+    work-groups took 1.7-3 times)."""
+    import torch
+    from npu_sparse_attn_sharedkv_int8 import PreparedAttention, SharedKVCase
+    capacity = 2048
+    made = DeviceCase(94, ratio, [live], [length])
+    eager = PreparedAttention(made.dev, made.ori_scale, made.cmp_scale)
+    d = made.dev
+    q = torch.cat([d.q, d.q.new_zeros((capacity - live,) + d.q.shape[1:])])
+    both = lambda table: None if table is None else torch.cat([table, table])
+    whole = SharedKVCase(q=q, ori=d.ori, ori_block_table=both(d.ori_block_table),
+                         cu_q=torch.tensor([0, live, live], dtype=torch.int32, device="cuda"),
+                         seq_lens=torch.tensor([length, 0], dtype=torch.int32, device="cuda"), sink=d.sink, cmp=d.cmp,
+                         cmp_block_table=both(d.cmp_block_table), cmp_indices=None, ratio=ratio, window=d.window,
+                         softmax_scale=d.softmax_scale)
+    op = PreparedAttention(whole, made.ori_scale, made.cmp_scale)
+    assert op.splits == 1
+    fill = torch.empty_like(op.out[live:])
+    took, alone, zero = microseconds(op.run), microseconds(eager.run), microseconds(fill.zero_)
+    print(f"[padded] ratio {ratio}, {live} of {capacity} at {length}: {took:.1f} us, eager {alone:.1f}, fill {zero:.1f}",
+          file=sys.stderr, flush=True)
+    assert took <= 1.5 * (alone + zero)
