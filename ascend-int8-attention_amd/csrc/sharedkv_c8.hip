@@ -514,11 +514,11 @@ __device__ __forceinline__ void fold_row(const __amdgpu_buffer_rsrc_t states, in
 // multiple of 8) with `items` work items.
 // TIGHT: nothing derived from the thread is held in a register from before
 // the row codes on (inside c8_chunk, whose scalar spills take registers).
-template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT, bool RESID, bool TIGHT>
+template <int RATIO, bool DEBUG, bool SLOTS, bool ANYH, bool STREAM, bool JOINT, bool RESID, bool TIGHT, class Args>
 __device__ __forceinline__ void
 attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint64_t cmp_indices,
                const uint32_t batch_arg, const uint32_t topk_arg, const uint32_t heads_arg, const uint32_t splits,
-               const uint32_t rows_arg, const uint32_t grid, const SharedKVArgs &p, const SharedKVDebug &dbg,
+               const uint32_t rows_arg, const uint32_t grid, const Args &p, const SharedKVDebug &dbg,
                const uint32_t fused, const uint32_t items, const uint32_t block, int tid)
 {
     int lane = tid & 63, wave = tid >> 6;
@@ -3046,6 +3046,12 @@ __device__ __forceinline__ void dma16_at(uint64_t base, uint32_t offset, uint32_
 // decides again with the live one.
 constexpr uint32_t CHUNK_ROUND = CHUNK_ROWS * PLAN_CUS, ROWS_ROUND = 2 * PLAN_CUS;
 constexpr uint32_t CHUNK_MIN_C128 = 768, CHUNK_REQUEST_TOKENS = 16;
+// Rows of a request in an octet up to which they are taken whole where the
+// octets' requests are spread over the work-groups (an octet costs 10 us
+// window-only and 6 us a tile for one row as for eight, c8_attention 5.4 and
+// 2): 1984 tokens of a chunk and 64 one-token requests, window-only 28 -> 23.5
+// us; 800 tokens and 40 C128 requests of 60-128 K 51 -> 32 us.
+constexpr int SHORT_TAIL = 2;
 
 // `rows` rows of eight heads of `tokens` query tokens and `batch` requests
 // take `rounds` rounds of octets; `own`: the rows as c8_rows counts them.
@@ -3058,11 +3064,25 @@ __host__ __device__ constexpr bool chunk_pays(int ratio, uint32_t tokens, uint32
     return ratio == 1 && (uint64_t)rounds * (WIDE ? 2 : 3) <= ((uint64_t)own + ROWS_ROUND - 1) / ROWS_ROUND;
 }
 
+// c8_chunk's kernel arguments as they lie in the kernel argument segment.
+struct ChunkKernelArgs {
+    uint64_t cu_q, seq_lens, q_base;
+    uint32_t batch, rows, heads;
+    SharedKVArgs args;
+    uint32_t fused;
+};
+// Read from there when they are used, whatever was read before.
+__device__ __forceinline__ const auto &chunk_kernel_args()
+{
+    auto at = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(at));
+    return *(const __attribute__((address_space(4))) ChunkKernelArgs *)at;
+}
+
 template <int RATIO, bool ANYH, bool RESID>
 __global__ void __launch_bounds__(THREADS, 1)
 c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, const uint32_t batch_arg,
-         const uint32_t rows_arg, const uint32_t grid, const uint32_t heads_arg, const SharedKVArgs p,
-         const uint32_t fused)
+         const uint32_t rows_arg, const uint32_t heads_arg, const SharedKVArgs p, const uint32_t fused)
 {
     static_assert(RATIO == 1 || RATIO == 128, "window-only and C128 launches");
     __shared__ alignas(16) uint8_t lds[sizeof(ChunkShared) > sizeof(Shared) ? sizeof(ChunkShared) : sizeof(Shared)];
@@ -3087,7 +3107,8 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
 
     // Work: octet o holds rows 8 o .. 8 o + 7 of the launch; XCD x takes a
     // contiguous eighth of them.
-    const int x = (int)(blockIdx.x & 7u), slot = (int)(blockIdx.x >> 3), per_xcd = (int)(grid >> 3);
+    constexpr int per_xcd = PLAN_CUS / 8;   // of the launch's PLAN_CUS work-groups
+    const int x = (int)(blockIdx.x & 7u), slot = (int)(blockIdx.x >> 3);
     int octets = (rows_cap + CHUNK_ROWS - 1) / CHUNK_ROWS;
     auto first_octet = [&](int xcd) { return (int)((int64_t)xcd * octets / 8); };
     int o = first_octet(x) + slot;
@@ -3130,9 +3151,11 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
         for (int h = 0; h < hlive; ++h) reinterpret_cast<v4i *>(out)[64 * h + lane] = v4i{0, 0, 0, 0};
         if (p.lse && lane < hlive) reinterpret_cast<float *>(p.lse)[(int64_t)t * H + hbase + lane] = 0.0f;
     };
-    if (live_tokens * HG < rows_cap) {
+    const int live_rows = live_tokens * HG;
+    bool whole = false, plan = false;   // every row by itself; with c8_attention's device plan
+    if (live_rows < rows_cap) {
         // Graph padding: its rows are zero (attention_impl.h:443-460).
-        for (int row = live_tokens * HG + (int)blockIdx.x * CHUNK_ROWS + wave; row < rows_cap; row += (int)grid * CHUNK_ROWS) {
+        for (int row = live_rows + (int)blockIdx.x * CHUNK_ROWS + wave; row < rows_cap; row += PLAN_CUS * CHUNK_ROWS) {
             const int h = ANYH ? HEADS * (row % HG) : 0;
             zero_row(ANYH ? row / HG : row, h, ANYH ? (H - h < HEADS ? H - h : HEADS) : HEADS);
         }
@@ -3143,61 +3166,63 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
             // host, over this launch's work-groups), unless every row is a
             // joint row.
             const int longest = longest_live(cu, lens, live_batch);
-            const int live_rows = live_tokens * HG, tiles = 1 + (longest / RATIO + N - 1) / N;
-            const bool plan =
-                fused && tiles > 1 && PLAN_CUS / live_rows > 1 && !(resid && longest / RATIO <= N);
+            const int tiles = 1 + (longest / RATIO + N - 1) / N;
+            plan = fused && tiles > 1 && PLAN_CUS / live_rows > 1 && !(resid && longest / RATIO <= N);
             // Otherwise the launch rule on the live shape: octets or, where an
             // eager launch of the live rows would not come here,
             // c8_attention's rows, one work-group each in turn.
-            if (plan || !chunk_pays<!RESID>(RATIO, live_tokens, live_batch, live_rows, live_rows, 0)) {
-                __builtin_amdgcn_s_setprio(0);
-                const uint32_t of_rows = plan ? rows_arg : (uint32_t)live_rows;
-                const uint32_t groups = plan ? grid : ((uint32_t)live_rows + 7u) & ~7u;
-                const uint32_t items = of_rows < groups ? of_rows : groups;
-                for (uint32_t block = blockIdx.x; block < groups; block += grid) {
-                    int thread = (int)threadIdx.x;   // opaque: no per-lane value is held across the rows
-                    asm volatile("" : "+v"(thread));
-                    attention_item<RATIO, false, false, ANYH, false, RESID, RESID, true>(
-                        *reinterpret_cast<Shared *>(lds), cu_q, seq_lens, q_base, 0, batch_arg, 0, heads_arg, 1, of_rows,
-                        groups, p, SharedKVDebug{0, 0, 0, 0, 0, 0, 0}, fused, items, block, thread);
-                    __syncthreads();
-                }
-                return;
-            }
+            whole = plan || !chunk_pays<!RESID>(RATIO, live_tokens, live_batch, live_rows, live_rows, 0);
         }
         // The octets of the live rows are spread over the XCDs instead.
-        octets = (live_tokens * HG + CHUNK_ROWS - 1) / CHUNK_ROWS;
-        o = first_octet(x) + slot;
-        load_row();
+        if (!whole) {
+            octets = (live_rows + CHUNK_ROWS - 1) / CHUNK_ROWS;
+            o = first_octet(x) + slot;
+            load_row();
+        }
     }
-    // Octets that straddle requests.  A request that starts inside an octet
-    // is a tail: `tails` of them, `crowded` if some octet holds two.
+    // Octets that straddle requests.  A request that starts inside an octet,
+    // or is short there, is a tail: `tails` of them, `crowded` if two requests
+    // start inside some octet.
     // Work-groups that would have nothing to do in the last round of octets
     // take the tails, one each, if they suffice or an octet is crowded (then
     // further rounds take the rest).  Otherwise an octet takes its two
     // requests at once (`pairs`, below).
+    // Tails of at most SHORT_TAIL rows (decode requests beside prefill chunks)
+    // are taken whole.
+    auto inside = [&](int c0) { return c0 * HG % CHUNK_ROWS != 0; };
+    auto octet_of = [&](int token) { return token * HG / CHUNK_ROWS; };
+    // Rows in its first octet of a request's tokens c0 .. c1 - 1, 0 if they are not short.
+    auto short_rows = [&](int c0, int c1) {
+        const int past = CHUNK_ROWS * octet_of(c0) + CHUNK_ROWS, end = (c1 < live_tokens ? c1 : live_tokens) * HG;
+        const int rows = (end < past ? end : past) - c0 * HG;
+        return HG <= SHORT_TAIL && rows <= SHORT_TAIL ? rows : 0;
+    };
     auto is_tail = [&](int c0, int c1) {
-        return c0 >= 0 && c0 < live_tokens && c1 > c0 && c0 * HG % CHUNK_ROWS != 0;
+        return c0 >= 0 && c0 < live_tokens && c1 > c0 && (inside(c0) || short_rows(c0, c1));
     };
     int tails = 0;
     bool crowded = false;
     auto count_tails = [&](int c0, int c1, bool there) {
         const bool mine = there && is_tail(c0, c1);
         tails += __popcll(__ballot(mine));
-        crowded |= __ballot(mine && c1 < live_tokens && c1 * HG / CHUNK_ROWS == c0 * HG / CHUNK_ROWS) != 0;
+        crowded |= __ballot(mine && inside(c0) && c1 < live_tokens && octet_of(c1) == octet_of(c0)) != 0;
     };
-    count_tails(my_cu0, my_cu1, (tid & 63) < live_batch);
-    for (int b0 = 64; b0 < live_batch; b0 += 64) {
-        const int b = b0 + (tid & 63) < live_batch ? b0 + (tid & 63) : live_batch - 1;
-        count_tails(cu[b], cu[b + 1], b0 + (tid & 63) < live_batch);
+    if (live_batch > 1) {
+        count_tails(my_cu0, my_cu1, (tid & 63) < live_batch);
+        for (int b0 = 64; b0 < live_batch; b0 += 64) {
+            const int b = b0 + (tid & 63) < live_batch ? b0 + (tid & 63) : live_batch - 1;
+            count_tails(cu[b], cu[b + 1], b0 + (tid & 63) < live_batch);
+        }
     }
-    int idle = 0, my_idle = -1;   // work-groups without an octet in their XCD's last round, and this one's number
-    for (int xcd = 0; xcd < 8; ++xcd) {
-        const int mine = first_octet(xcd + 1) - first_octet(xcd), used = mine % per_xcd;
-        if (mine && !used) continue;
-        if (xcd == x && slot >= used) my_idle = idle + slot - used;
-        idle += per_xcd - used;
-    }
+    // Work-groups without an octet in their XCD's last round, and this one's
+    // number among them: an XCD holds octets / 8 octets or one more, the
+    // latter for x * (octets % 8) / 8 of the XCDs before x.
+    auto idle_of = [](int held) { return held ? -held & (per_xcd - 1) : per_xcd; };
+    const int fewer = idle_of(octets >> 3), more_held = idle_of((octets >> 3) + 1), extra = octets & 7;
+    const int idle = (8 - extra) * fewer + extra * more_held;
+    const int before = x * extra >> 3, mine = first_octet(x + 1) - first_octet(x), mine_idle = idle_of(mine);
+    const int my_idle =
+        slot >= per_xcd - mine_idle ? (x - before) * fewer + before * more_held + slot - (per_xcd - mine_idle) : -1;
     const bool split = tails <= idle || crowded;
     // Token at which tail `e` starts.
     auto tail_start = [&](int e) {
@@ -3218,22 +3243,30 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
         return -1;
     };
     const int past_octet = first_octet(x + 1);
-    int first = ANYH ? CHUNK_ROWS * o / HG : CHUNK_ROWS * o;
+    auto token_of = [&](int octet) { return ANYH ? CHUNK_ROWS * octet / HG : CHUNK_ROWS * octet; };
+    int first = token_of(o);
     bool tail = false;
-    int next_tail = my_idle >= 0 ? my_idle : idle + (int)blockIdx.x;
-    // The work-group's next tail; false when there is none.
+    const int first_tail = my_idle >= 0 ? my_idle : idle + (int)blockIdx.x;
+    int next_tail = first_tail;
+    auto after = [&](int e) { return e < idle ? idle + (int)blockIdx.x : e + PLAN_CUS; };
+    // The work-group's next tail that is not short; false when there is none.
+    // (The short ones follow the octets.)
     auto take_tail = [&]() {
-        if (!split || next_tail >= tails) return false;
-        first = tail_start(next_tail);
-        next_tail = next_tail < idle ? idle + (int)blockIdx.x : next_tail + (int)grid;
-        tail = true;
-        o = first * HG / CHUNK_ROWS;
-        load_row();
-        const int c1 = request_of(first).c1;
-        stop = c1 < stop ? c1 : stop;
-        return true;
+        if (!split) return false;
+        for (; next_tail < tails; next_tail = after(next_tail)) {
+            first = tail_start(next_tail);
+            const int c1 = request_of(first).c1;
+            if (short_rows(first, c1)) continue;
+            next_tail = after(next_tail);
+            tail = true;
+            o = octet_of(first);
+            load_row();
+            stop = c1 < stop ? c1 : stop;
+            return true;
+        }
+        return false;
     };
-    if (o >= past_octet && !take_tail()) return;
+    bool more = !whole && (o < past_octet || take_tail());
     *reinterpret_cast<f32x2 *>(&s.scale[tid >> 8][(tid & 255) * 2]) = scale_pair;
 
     // The next octet or tail of the work-group, its rows' Q on its way; false
@@ -3242,21 +3275,29 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
         if (tail || o + per_xcd >= past_octet) return take_tail();
         o += per_xcd;
         load_row();
-        first = ANYH ? CHUNK_ROWS * o / HG : CHUNK_ROWS * o;
+        first = token_of(o);
         return true;
     };
 
-    for (bool more = true; more;) {
+    const SharedKVArgs &launch = p;
+    auto args_again = [&]() -> const auto & {
+        if constexpr (RATIO == 128) return chunk_kernel_args().args;
+        else return launch;
+    };
+    while (more) {
         {
             if (first >= stop || first >= live_tokens) {
                 more = next_item();
                 continue;
             }
-            const int start = ANYH ? CHUNK_ROWS * o / HG : CHUNK_ROWS * o;   // the octet's first token
             // Per-lane values derive from an opaque copy of the lane index, so
-            // that none is held in a register across the loop.
+            // that none is held in a register across the loop, and C128 reads
+            // the arguments again (held, they send 500 scalar reads through
+            // lanes of vector registers: 44.1 us on three requests of 662 rows
+            // on average, and 43.1 so).
             int lane = tid & 63;
             asm volatile("" : "+v"(lane));
+            const auto &p = args_again();
             const int g = lane >> 4, n = lane & 15;
             // Tokens of no live request and negative positions (reference.py:
             // 104-105 rejects them) are zero.
@@ -3282,8 +3323,8 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
                 tiles[i] = (all_rows[i] + N - 1) / N;
             };
             segment(0, first, r0);
-            if (split && !tail && first != start && first == r0.c0) {   // a tail, taken elsewhere
-                first = past[0];
+            if (split && !tail && first == r0.c0 && (first != token_of(o) || short_rows(first, r0.c1))) {
+                first = past[0];   // a tail, taken elsewhere
                 continue;
             }
             batch[1] = back[1] = from[1] = past[1] = lo0[1] = span[1] = all_rows[1] = tiles[1] = 0;
@@ -3497,7 +3538,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
                 const int r0 = shift + 8 * gx + (nx >> 1), f = r0 & 15;
                 const lds_i8 *at = tb + r0 * D + 8 * (nx & 1);
                 const float *sc = s.scale[kind] + nx;
-constexpr int PC = 2;
+                constexpr int PC = 2;
                 // Column chunk jc (16 PC columns): the next chunk's reads are in flight
                 // during its MFMAs and epilogue.
                 v2i bb[2][4 * PC];
@@ -3733,6 +3774,39 @@ constexpr int PC = 2;
             }
         }
     }
+
+    // ---- rows taken whole: those of the launch, or the work-group's short tails ----
+    if (!whole && !(split && first_tail < tails && HG <= SHORT_TAIL)) return;
+    __builtin_amdgcn_s_setprio(0);
+    const uint32_t of_rows = plan ? (uint32_t)rows_cap : (uint32_t)live_rows;
+    const uint32_t groups = plan ? (uint32_t)PLAN_CUS : (of_rows + 7u) & ~7u;
+    const uint32_t items = of_rows < groups ? of_rows : groups;
+    uint32_t block = blockIdx.x;
+    int row = 0, past_row = 0, e = first_tail;
+    while (true) {
+        if (!whole) {
+            for (; row >= past_row && e < tails; e = after(e)) {
+                const int c0 = tail_start(e);
+                row = c0 * HG;
+                past_row = row + short_rows(c0, request_of(c0).c1);
+            }
+            if (row >= past_row) break;
+            block = (uint32_t)row % (groups / 8) * 8 + (uint32_t)row / (groups / 8);   // of work item `row`
+            ++row;
+        } else if (block >= groups) {
+            break;
+        }
+        __syncthreads();   // every wave is done with the row or octet before
+        // Opaque: nothing derived from the thread or the kernel arguments is
+        // held in registers for this from before the octets on.
+        int thread = (int)threadIdx.x;
+        asm volatile("" : "+v"(thread));
+        const auto &k = chunk_kernel_args();
+        attention_item<RATIO, false, false, ANYH, false, RATIO == 128 && RESID, RESID, true>(
+            *reinterpret_cast<Shared *>(lds), k.args.cuQ, k.args.seqLens, k.args.q, 0, k.args.batch, 0, k.args.heads, 1, of_rows,
+            groups, k.args, SharedKVDebug{0, 0, 0, 0, 0, 0, 0}, k.fused, items, block, thread);
+        block += PLAN_CUS;
+    }
 }
 
 // ---- INT8 cache writer (cache_write.cpp:9-88): one wave per update row ----
@@ -3892,9 +3966,8 @@ void launch_variant(hipStream_t stream, const SharedKVArgs *a, const SharedKVDeb
     const uint32_t own = wide ? a->tokens * ((a->heads + WIDE_HEADS - 1) / WIDE_HEADS) : rows;
     const uint32_t rounds = (uint32_t)(((uint64_t)rows + CHUNK_ROUND - 1) / CHUNK_ROUND);
     if (!DEBUG && !slots && splits == 1 && chunk_pays<wide>((int)a->ratio, a->tokens, a->batch, rows, own, rounds)) {
-        const uint32_t cus = (uint32_t)PLAN_CUS;
-        hipLaunchKernelGGL((a->ratio == 1 ? &c8_chunk<1, ANYH, RESID> : &c8_chunk<128, ANYH, RESID>), dim3(cus), dim3(THREADS), 0, stream,
-                           a->cuQ, a->seqLens, a->q, a->batch, rows, cus, a->heads, *a, fused);
+        hipLaunchKernelGGL((a->ratio == 1 ? &c8_chunk<1, ANYH, RESID> : &c8_chunk<128, ANYH, RESID>), dim3(PLAN_CUS),
+                           dim3(THREADS), 0, stream, a->cuQ, a->seqLens, a->q, a->batch, rows, a->heads, *a, fused);
         return;
     }
     // One-partition C4 and window-only launches of more rows than CUs

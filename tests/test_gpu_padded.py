@@ -1,13 +1,15 @@
-"""Prefill launches at a graph's capacity with few live rows: the kernel that
-the capacity selects (c8_chunk) runs them as the kernel that an eager launch of
-the live rows would run, bit-exact with the oracle and in about its time."""
+"""Launches that the capacity or the average request sends to c8_chunk and whose
+live rows another kernel takes in less time: few live rows in a graph's prefill
+capacity, and a full prefill chunk with many one-token requests beside it.
+c8_chunk runs such rows whole, as c8_attention would, bit-exact with the oracle
+and in about their time."""
 import sys
 
 import numpy as np
 import pytest
 
 from tests import workloads
-from tests.device_cases import DeviceCase, joint_flags, run_hip, run_oracle
+from tests.device_cases import DeviceCase, joint_flags, query_subcase, run_hip, run_oracle
 from tests.test_gpu_chunk import padded
 
 pytestmark = pytest.mark.gpu
@@ -20,23 +22,32 @@ CASES = [
     ("joint", 128, [290, 40], [3000, 700], 8, 900),                # every row joint, two passes
     ("head_groups", 128, [150, 40], [17000, 2500], 20, 400),       # 570 rows of three groups
     ("many_requests", 128, [4] * 210, list(range(300, 300 + 210 * 90, 90)), 8, 2600),   # 840 rows, four a request
+    ("window_mixed", 1, [1] * 64 + [1984], list(range(90, 90 + 64 * 40, 40)) + [2500], 8, 0),   # 56 tails of 256 octets
+    ("mixed", 128, [1] * 20 + [801] + [2] * 10, list(range(200, 200 + 20 * 900, 900)) + [17100] + [16500, 40] * 5, 8, 3),
+    ("mixed_groups", 128, [600] + [1] * 30, [16900] + list(range(100, 100 + 30 * 700, 700)), 16, 0),   # two rows a token
+    ("window_mixed_groups", 1, [901] + [1] * 40, [1300] + list(range(1, 1 + 40 * 50, 50)), 16, 2),
 ]
 
 
 @pytest.mark.parametrize("name,ratio,queries,lengths,heads,pad", CASES, ids=[c[0] for c in CASES])
 def test_padded_launch_matches_oracle(name, ratio, queries, lengths, heads, pad):
+    from npu_sparse_attn_sharedkv_int8 import c8_attention
     print(f"[padded] {name}", file=sys.stderr, flush=True)
     case = workloads.make_case(93, ratio, queries, lengths, heads=heads)
-    launch = padded(case, pad)
+    launch = padded(case, pad) if pad else case
     rows, live = launch["q"].shape[0] * ((heads + 7) // 8), int(case["cu_q"][-1])
     assert (rows > 1024 if ratio == 1 else rows > 768) and launch["q"].shape[0] >= 16 * len(launch["seq_lens"])
     out, lse, op = run_hip(launch, splits=1)
     assert op.device_splits() == 1
     assert not out[live:].any() and not lse[live:].any(), "padding rows are not zero"
-    ref, ref_lse, _ = run_oracle(case, 1, joint=joint_flags(launch, 1))
-    diff = out[:live] != ref
+    dead = c8_attention.keyless_tokens(case["cu_q"], case["seq_lens"], live)
+    keep = [t for t in range(live) if not dead[t]]
+    assert not out[[t for t in range(live) if dead[t]]].any(), "keyless rows are not zero"
+    sub = case if len(keep) == live else query_subcase(case, keep)
+    ref, ref_lse, _ = run_oracle(sub, 1, joint=joint_flags(launch, 1))
+    diff = out[keep] != ref
     assert not diff.any(), f"{int(diff.sum())} BF16 mismatches, rows {sorted(set(np.argwhere(diff)[:, 0]))[:8]}"
-    np.testing.assert_allclose(lse[:live], ref_lse, rtol=0, atol=2e-6)
+    np.testing.assert_allclose(lse[keep], ref_lse, rtol=0, atol=2e-6)
 
 
 def microseconds(call, calls=50, rounds=7):
@@ -81,3 +92,19 @@ def test_padded_launch_takes_the_time_of_its_live_rows(ratio, live, length):
     print(f"[padded] ratio {ratio}, {live} of {capacity} at {length}: {took:.1f} us, eager {alone:.1f}, fill {zero:.1f}",
           file=sys.stderr, flush=True)
     assert took <= 1.5 * (alone + zero)
+
+
+def test_chunk_with_decode_requests_takes_the_time_of_its_parts():
+    """2048 window-only tokens, 64 of them requests of one token: octets would
+    need a second round for those (1.18 times the two parts' own launches, here
+    0.98)."""
+    from npu_sparse_attn_sharedkv_int8 import PreparedAttention
+    parts = [([1] * 64, list(range(1000, 1000 + 64 * 400, 400))), ([1984], [32768])]
+    whole = tuple(parts[0][i] + parts[1][i] for i in range(2))
+    times = []
+    for queries, lengths in (whole, *parts):
+        made = DeviceCase(95, 1, queries, lengths)
+        op = PreparedAttention(made.dev, made.ori_scale, made.cmp_scale)
+        times.append(microseconds(op.run))
+    print(f"[padded] mixed: {times[0]:.1f} us, its parts {times[1]:.1f} and {times[2]:.1f}", file=sys.stderr, flush=True)
+    assert times[0] <= 1.1 * (times[1] + times[2])
