@@ -3046,6 +3046,11 @@ __device__ __forceinline__ void dma16_at(uint64_t base, uint32_t offset, uint32_
 // decides again with the live one.
 constexpr uint32_t CHUNK_ROUND = CHUNK_ROWS * PLAN_CUS, ROWS_ROUND = 2 * PLAN_CUS;
 constexpr uint32_t CHUNK_MIN_C128 = 768, CHUNK_REQUEST_TOKENS = 16;
+// Padded window-only launches take up to CHUNK_WHOLE live rows whole, as
+// c8_attention takes them (of 2048: 256 live rows 11.2 us and 21.0 as octets,
+// 512 14.9 and 19.9; each 256 more cost 4 us, octets of up to 2048 rows stay
+// at 19-20).
+constexpr int CHUNK_WHOLE = 2 * PLAN_CUS;
 // Rows of a request in an octet up to which they are taken whole where the
 // octets' requests are spread over the work-groups (an octet costs 10 us
 // window-only and 6 us a tile for one row as for eight, c8_attention 5.4 and
@@ -3172,6 +3177,8 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
             // eager launch of the live rows would not come here,
             // c8_attention's rows, one work-group each in turn.
             whole = plan || !chunk_pays<!RESID>(RATIO, live_tokens, live_batch, live_rows, live_rows, 0);
+        } else {
+            whole = live_rows <= CHUNK_WHOLE;
         }
         // The octets of the live rows are spread over the XCDs instead.
         if (!whole) {

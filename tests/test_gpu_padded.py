@@ -22,6 +22,12 @@ CASES = [
     ("joint", 128, [290, 40], [3000, 700], 8, 900),                # every row joint, two passes
     ("head_groups", 128, [150, 40], [17000, 2500], 20, 400),       # 570 rows of three groups
     ("many_requests", 128, [4] * 210, list(range(300, 300 + 210 * 90, 90)), 8, 2600),   # 840 rows, four a request
+    ("window", 1, [300, 9], [17000, 700], 8, 1300),                # some work-group of an XCD with one row of its two
+    ("window_one_row", 1, [1], [50], 8, 1300),
+    ("window_passes", 1, [600, 300], [900, 4000], 8, 400),         # 900 rows over 512 half work-groups
+    ("window_keyless", 1, [200, 4, 90], [198, 1, 300], 8, 1300),   # negative positions
+    ("window_groups", 1, [100, 33], [3000, 50], 20, 700),          # rows of sixteen heads and of four
+    ("window_four_heads", 1, [61], [2000], 4, 1300),
     ("window_mixed", 1, [1] * 64 + [1984], list(range(90, 90 + 64 * 40, 40)) + [2500], 8, 0),   # 56 tails of 256 octets
     ("mixed", 128, [1] * 20 + [801] + [2] * 10, list(range(200, 200 + 20 * 900, 900)) + [17100] + [16500, 40] * 5, 8, 3),
     ("mixed_groups", 128, [600] + [1] * 30, [16900] + list(range(100, 100 + 30 * 700, 700)), 16, 0),   # two rows a token
@@ -66,7 +72,8 @@ def microseconds(call, calls=50, rounds=7):
     return sorted(times)[rounds // 2]
 
 
-@pytest.mark.parametrize("ratio,live,length", [(128, 40, 6000), (128, 200, 32768), (128, 200, 131072)])
+@pytest.mark.parametrize("ratio,live,length", [(128, 40, 6000), (128, 200, 32768), (128, 200, 131072),
+                                               (1, 40, 8192), (1, 512, 8192)])
 def test_padded_launch_takes_the_time_of_its_live_rows(ratio, live, length):
     """A launch of 2048 query tokens with `live` live ones takes no more than
     1.5 times an eager launch of those and a fill of the padding's outputs
