@@ -3214,7 +3214,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
         tails += __popcll(__ballot(mine));
         crowded |= __ballot(mine && inside(c0) && c1 < live_tokens && octet_of(c1) == octet_of(c0)) != 0;
     };
-    if (live_batch > 1) {
+    if (live_batch > 1 || uni(my_cu0) > 0) {   // (a lone request from token 0 on starts no octet late)
         count_tails(my_cu0, my_cu1, (tid & 63) < live_batch);
         for (int b0 = 64; b0 < live_batch; b0 += 64) {
             const int b = b0 + (tid & 63) < live_batch ? b0 + (tid & 63) : live_batch - 1;

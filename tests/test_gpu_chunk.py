@@ -74,6 +74,22 @@ def test_chunk_launch_matches_oracle(name, ratio, queries, lengths, heads, pad):
     np.testing.assert_allclose(lse[keep], ref_lse, rtol=0, atol=2e-6)
 
 
+@pytest.mark.parametrize("ratio,queries,length,before", [(1, 1097, 1300, 3), (128, 900, 17300, 13), (128, 2, 17000, 1200)])
+def test_tokens_before_the_first_request(ratio, queries, length, before):
+    """One request that starts at token `before`, inside an octet or short: its
+    rows are computed and the tokens of no request are zero."""
+    case = workloads.make_case(96, ratio, [queries], [length])
+    nan = np.full((before,) + case["q"].shape[1:], 0x7FC0, np.uint16)
+    launch = dict(case, q=np.concatenate([nan, case["q"]]), cu_q=case["cu_q"] + np.int32([before, before]))
+    assert launch["cu_q"].dtype == np.int32
+    say(f"[chunk] {before} tokens before the first request, ratio {ratio}")
+    out, lse, op = run_hip(launch, splits=1)
+    assert not out[:before].any() and not lse[:before].any()
+    ref, ref_lse, _ = run_oracle(case, 1, joint=joint_flags(launch, 1))
+    assert (out[before:] == ref).all()
+    np.testing.assert_allclose(lse[before:], ref_lse, rtol=0, atol=2e-6)
+
+
 @pytest.mark.parametrize("ratio", [1, 128])
 def test_unreadable_pages_equal_the_general_path(ratio):
     """Block-table entries past the pool (window) and negative ones
