@@ -90,6 +90,50 @@ def test_tokens_before_the_first_request(ratio, queries, length, before):
     np.testing.assert_allclose(lse[before:], ref_lse, rtol=0, atol=2e-6)
 
 
+ROUNDS = [   # more than 256 octets: a work-group takes several, one after the other
+    ("partial", 1, [2601], [2601], 8, 0),                                # a last round of 70 octets, the last of one row
+    ("partial_c128", 128, [2100], [17600], 8, 0),
+    ("three", 1, [4300], [5000], 8, 0),
+    ("three_c128", 128, [4300], [9000], 8, 0),
+    ("joint_boundary", 128, [2200], [17200], 8, 0),                      # joint rows first, rows of two tiles after them
+    ("tails", 128, [1003, 900, 203], [17000, 3000, 9100], 8, 0),         # taken by the last round's idle work-groups
+    ("full_pairs", 1, [1501, 1302, 1293], [1600, 4000, 1293], 8, 0),     # 512 octets, none idle: two requests at once
+    ("full_pairs_c128", 128, [1501, 1302, 1293], [17600, 3000, 9000], 8, 0),
+    ("mixed", 128, [1000] + [1] * 20 + [1203], [17000] + list(range(200, 200 + 20 * 900, 900)) + [2500], 8, 0),
+    ("head_groups", 128, [700, 201], [17000, 2500], 20, 0),              # 2703 rows of three groups
+    ("padded", 1, [2500, 301], [2600, 900], 8, 800),
+]
+
+
+@pytest.mark.parametrize("name,ratio,queries,lengths,heads,pad", ROUNDS, ids=[c[0] for c in ROUNDS])
+def test_several_rounds_match_oracle(name, ratio, queries, lengths, heads, pad):
+    say(f"[chunk] rounds: {name}")
+    case = workloads.make_case(97, ratio, queries, lengths, heads=heads)
+    launch = padded(case, pad) if pad else case
+    live = int(case["cu_q"][-1])
+    groups = (heads + 7) // 8
+    assert live * groups > (2560 if ratio == 1 else 2048) and launch["q"].shape[0] >= 16 * len(launch["seq_lens"])
+    out, lse, op = run_hip(launch, splits=1)
+    assert op.device_splits() == 1
+    assert not out[live:].any() and not lse[live:].any(), "padding rows are not zero"
+    ref, ref_lse, _ = run_oracle(case, 1, joint=joint_flags(launch, 1))
+    diff = out[:live] != ref
+    assert not diff.any(), f"{int(diff.sum())} BF16 mismatches, rows {sorted(set(np.argwhere(diff)[:, 0]))[:8]}"
+    np.testing.assert_allclose(lse[:live], ref_lse, rtol=0, atol=2e-6)
+
+
+@pytest.mark.parametrize("ratio", [1, 128])
+def test_unreadable_pages_of_the_first_round(ratio):
+    """Masked window rows in a work-group's first octet and none in its second."""
+    case = workloads.make_case(98, ratio, [2900], [3100])
+    case["ori"].table[0, 20] = case["ori"].pages + 3   # logical rows 640-671: query rows 440-598
+    say(f"[chunk] unreadable pages of the first round, ratio {ratio}")
+    out, lse, op = run_hip(case, splits=1)
+    rows = list(range(430, 720, 2))   # octets 55-74 of XCD 1, and 77-89, the second of its work-groups
+    ref, ref_lse, few = run_hip(query_subcase(case, rows), splits=1)
+    assert (out[rows] == ref).all() and (lse[rows] == ref_lse).all()
+
+
 @pytest.mark.parametrize("ratio", [1, 128])
 def test_unreadable_pages_equal_the_general_path(ratio):
     """Block-table entries past the pool (window) and negative ones
