@@ -305,9 +305,12 @@ __device__ __forceinline__ uint32_t low_bytes(float a, float b, float c, float d
     return ab | cd;
 }
 
-// num / den, correctly rounded, from the correctly rounded reciprocal r of
-// den: the FMA residual of the product corrects it (Markstein, 1990; den is
-// a softmax denominator, so no operand is subnormal).
+// num / den from the correctly rounded reciprocal r of den: the FMA residual
+// of the product corrects it (Markstein, 1990).  Correctly rounded where the
+// residual is exact and the quotient normal: den is a softmax denominator, at
+// least 1 and far below 2^24, so numerators of 2^-100 and up will do (in
+// subnormal quotients a third of the FP32 results are off by one unit).
+constexpr float TINY = 0x1p-100f;
 __device__ __forceinline__ float div_by(float num, float den, float r)
 {
     const float q = num * r;
@@ -315,6 +318,34 @@ __device__ __forceinline__ float div_by(float num, float den, float r)
     // finite number, which leaves the infinity as it is.
     const float e = __builtin_amdgcn_fmed3f(__builtin_fmaf(-q, den, num), -3.0e38f, 3.0e38f);
     return __builtin_fmaf(e, r, q);
+}
+// Whether a numerator of the wave is smaller than that (or zero).
+template <int HH, int K>
+__device__ __forceinline__ bool any_tiny(const float (&num)[HH][K])
+{
+    float least = fabsf(num[0][0]);
+#pragma unroll
+    for (int k = 1; k < HH * K; ++k) least = fminf(least, fabsf(num[k / K][k % K]));
+    return __ballot(least < TINY) != 0;
+}
+// Then the wave divides and leaves the quotients to be divided by 1.
+template <int HH, int K>
+__device__ __forceinline__ void divide_tiny(float (&num)[HH][K], float (&den)[HH], float (&r)[HH])
+{
+    if (__builtin_expect(!any_tiny(num), 1)) return;
+    // Not unrolled, by rotation (a launch of one C128 row: 7.9 us without this,
+    // 8.1 with straight-line code, 7.95 with this).
+#pragma nounroll
+    for (int i = 0; i < K; ++i)
+#pragma unroll
+        for (int hh = 0; hh < HH; ++hh) {
+            const float q = num[hh][0] / den[hh];
+#pragma unroll
+            for (int k = 1; k < K; ++k) num[hh][k - 1] = num[hh][k];
+            num[hh][K - 1] = q;
+        }
+#pragma unroll
+    for (int hh = 0; hh < HH; ++hh) den[hh] = r[hh] = 1.0f;
 }
 
 // P codes of keys 64 kb + 16 g .. + 15 in the MFMA A layout, from a tile's
@@ -404,23 +435,24 @@ __device__ __forceinline__ void fold_states(const __amdgpu_buffer_rsrc_t states,
         f[sp] = sk_expf_nonpos(ms[sp] - top);
         dsum = sp < S ? dsum + ds[sp] * f[sp] : dsum;
     }
-    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    float acc[1][8] = {};
 #pragma unroll
     for (int sp = 0; sp < MAXS; ++sp)
         if (sp < S) {
-            acc[0] = acc[0] + v0[sp].x * f[sp];
-            acc[1] = acc[1] + v0[sp].y * f[sp];
-            acc[2] = acc[2] + v0[sp].z * f[sp];
-            acc[3] = acc[3] + v0[sp].w * f[sp];
-            acc[4] = acc[4] + v1[sp].x * f[sp];
-            acc[5] = acc[5] + v1[sp].y * f[sp];
-            acc[6] = acc[6] + v1[sp].z * f[sp];
-            acc[7] = acc[7] + v1[sp].w * f[sp];
+            acc[0][0] = acc[0][0] + v0[sp].x * f[sp];
+            acc[0][1] = acc[0][1] + v0[sp].y * f[sp];
+            acc[0][2] = acc[0][2] + v0[sp].z * f[sp];
+            acc[0][3] = acc[0][3] + v0[sp].w * f[sp];
+            acc[0][4] = acc[0][4] + v1[sp].x * f[sp];
+            acc[0][5] = acc[0][5] + v1[sp].y * f[sp];
+            acc[0][6] = acc[0][6] + v1[sp].z * f[sp];
+            acc[0][7] = acc[0][7] + v1[sp].w * f[sp];
         }
-    const float r = 1.0f / dsum;
+    float by[1] = {dsum}, r[1] = {1.0f / dsum};
+    divide_tiny(acc, by, r);
     uint32_t w[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = pack_bf16(div_by(acc[2 * e], dsum, r), div_by(acc[2 * e + 1], dsum, r));
+    for (int e = 0; e < 4; ++e) w[e] = pack_bf16(div_by(acc[0][2 * e], by[0], r[0]), div_by(acc[0][2 * e + 1], by[0], r[0]));
     if (heads < HEADS && h >= heads) return;   // padding heads of the last group of eight
     *reinterpret_cast<v4i *>(out_row + h * D + col) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     if (lse_row && (tid & 63) == 0) lse_row[h] = top + logf(dsum);
@@ -449,7 +481,7 @@ __device__ __forceinline__ void fold_states_wide(const __amdgpu_buffer_rsrc_t st
 #pragma unroll
     for (int sp = 1; sp < (int)MAX_SPLITS; ++sp) top = sp < S ? fmaxf(top, ms[sp]) : top;
     float dsum = 0.0f;
-    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    float acc[1][8] = {};
 #pragma unroll
     for (int c = 0; c < (int)MAX_SPLITS; c += CHUNK) {
         if (c >= S) break;
@@ -467,20 +499,21 @@ __device__ __forceinline__ void fold_states_wide(const __amdgpu_buffer_rsrc_t st
             if (c + k < S) {
                 const float f = sk_expf_nonpos(ms[c + k] - top);
                 dsum = dsum + ds[k] * f;
-                acc[0] = acc[0] + v0[k].x * f;
-                acc[1] = acc[1] + v0[k].y * f;
-                acc[2] = acc[2] + v0[k].z * f;
-                acc[3] = acc[3] + v0[k].w * f;
-                acc[4] = acc[4] + v1[k].x * f;
-                acc[5] = acc[5] + v1[k].y * f;
-                acc[6] = acc[6] + v1[k].z * f;
-                acc[7] = acc[7] + v1[k].w * f;
+                acc[0][0] = acc[0][0] + v0[k].x * f;
+                acc[0][1] = acc[0][1] + v0[k].y * f;
+                acc[0][2] = acc[0][2] + v0[k].z * f;
+                acc[0][3] = acc[0][3] + v0[k].w * f;
+                acc[0][4] = acc[0][4] + v1[k].x * f;
+                acc[0][5] = acc[0][5] + v1[k].y * f;
+                acc[0][6] = acc[0][6] + v1[k].z * f;
+                acc[0][7] = acc[0][7] + v1[k].w * f;
             }
     }
-    const float r = 1.0f / dsum;
+    float by[1] = {dsum}, r[1] = {1.0f / dsum};
+    divide_tiny(acc, by, r);
     uint32_t w[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = pack_bf16(div_by(acc[2 * e], dsum, r), div_by(acc[2 * e + 1], dsum, r));
+    for (int e = 0; e < 4; ++e) w[e] = pack_bf16(div_by(acc[0][2 * e], by[0], r[0]), div_by(acc[0][2 * e + 1], by[0], r[0]));
     if (heads < HEADS && h >= heads) return;
     *reinterpret_cast<v4i *>(out_row + h * D + col) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     if (lse_row && (tid & 63) == 0) lse_row[h] = top + logf(dsum);
@@ -1462,14 +1495,15 @@ attention_item(Shared &s, const uint64_t cu_q, const uint64_t seq_lens, const ui
 
         if (folded == 1) {
             // ---- finalize (reference.py:317-323 with one partition) ----
+            float by[2] = {den[0], den[1]}, r[2] = {1.0f / den[0], 1.0f / den[1]};
+            divide_tiny(num, by, r);
 #pragma unroll
             for (int hh = 0; hh < 2; ++hh) {
                 const int h = 2 * g + hh;
                 if (ANYH && h >= hlive) continue;
-                const float r = 1.0f / den[hh];
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    out_row[h * D + c0 + 16 * j + n] = (uint16_t)pack_bf16(div_by(num[hh][j], den[hh], r), 0.0f);
+                    out_row[h * D + c0 + 16 * j + n] = (uint16_t)pack_bf16(div_by(num[hh][j], by[hh], r[hh]), 0.0f);
                 if (lse_row && wave == 0 && n == 0) lse_row[h] = mx[hh] + logf(den[hh]);
             }
             if (S > 1 && !fused && tid == 0)
@@ -2187,15 +2221,21 @@ c8_rows(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, con
         if (folded == 1) {
             // ---- finalize (reference.py:317-323 with one partition) ----
             const uint32_t pick = n & 1 ? 0x03020706u : 0x05040100u;
+            float by[NH], rden[NH];
+#pragma unroll
+            for (int hh = 0; hh < NH; ++hh) {
+                by[hh] = den[hh];
+                rden[hh] = 1.0f / den[hh];
+            }
+            divide_tiny(num, by, rden);
 #pragma unroll
             for (int hh = 0; hh < NH; ++hh) {
                 const int h = NH * g + hh;
-                const float rden = 1.0f / den[hh];
                 uint32_t *to = reinterpret_cast<uint32_t *>(out_row + h * D + c0) + 8 * (n & 1) + (n >> 1);
 #pragma unroll
                 for (int j = 0; j < 8; j += 2) {
                     // Lanes n and n ^ 1 exchange one column of two, so that each writes two neighbours.
-                    const uint32_t mine = pack_bf16(div_by(num[hh][j], den[hh], rden), div_by(num[hh][j + 1], den[hh], rden));
+                    const uint32_t mine = pack_bf16(div_by(num[hh][j], by[hh], rden[hh]), div_by(num[hh][j + 1], by[hh], rden[hh]));
                     const uint32_t other = (uint32_t)dpp_i<DPP_XOR1>((int)mine);
                     const uint32_t both = __builtin_amdgcn_perm(other, mine, pick);
                     if (!ANYH || h < hlive) __builtin_nontemporal_store(both, to + 8 * j);
@@ -3009,6 +3049,7 @@ constexpr int OUT_STRIDE = 2 * D + 32;               // LDS row stride of a head
 
 struct alignas(16) ChunkShared {
     float scale[2][D];                     // channel scales of the window / compressed cache
+    int8_t small_scale[CHUNK_ROWS];        // per wave: a scale it loaded is below 2^70 TINY
     int8_t bad[2][CHUNK_ROWS];             // per wave: some window row it copied lies on no readable page
     int8_t window_ok[2][CHUNK_UNION];      // union rows on a readable page
     int8_t p[CHUNK_ROWS][N * 16];          // P codes of each wave's row [key][MFMA row]
@@ -3275,6 +3316,8 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
     };
     bool more = !whole && (o < past_octet || take_tail());
     *reinterpret_cast<f32x2 *>(&s.scale[tid >> 8][(tid & 255) * 2]) = scale_pair;
+    if (RATIO == 1)
+        s.small_scale[wave] = __ballot(!(fminf(fabsf(scale_pair.x), fabsf(scale_pair.y)) >= 0x1p70f * TINY)) != 0;
 
     // The next octet or tail of the work-group, its rows' Q on its way; false
     // when there is none.
@@ -3755,17 +3798,31 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
             lds_barrier();   // the buffers are free
             if (active) {
                 int8_t *stage = s.buf[0] + wave * HEADS * OUT_STRIDE;
+                // As divide_tiny, unrolled (the rotation would cost a window-only
+                // launch 3.5 us, this 0.3).  A window-only numerator is one
+                // product, zero (0 * r is exact) or at least 2^-30 of its
+                // channel's scale.
+                const bool tiny = RATIO == 1 ? __ballot(s.small_scale[lane & (CHUNK_ROWS - 1)]) != 0 : any_tiny(num);
+                float by[2] = {den[0], den[1]};
+                if (__builtin_expect(tiny, 0)) {
+#pragma unroll
+                    for (int hh = 0; hh < 2; ++hh) {
+#pragma unroll
+                        for (int c = 0; c < 32; ++c) num[hh][c] = num[hh][c] / den[hh];
+                        by[hh] = 1.0f;
+                    }
+                }
 #pragma unroll
                 for (int hh = 0; hh < 2; ++hh) {
                     // Columns 16 c + n and 16 (c + 1) + n: lanes n and n ^ 1
                     // exchange one of them, so that each writes two neighbours
                     // (even lanes of block c, odd lanes of block c + 1).
-                    const float r = 1.0f / den[hh];
+                    const float r = 1.0f / by[hh];
                     const uint32_t pick = n & 1 ? 0x03020706u : 0x05040100u;
                     uint32_t *to = reinterpret_cast<uint32_t *>(stage + (2 * g + hh) * OUT_STRIDE) + 8 * (n & 1) + (n >> 1);
 #pragma unroll
                     for (int c = 0; c < 32; c += 2) {
-                        const uint32_t mine = pack_bf16(div_by(num[hh][c], den[hh], r), div_by(num[hh][c + 1], den[hh], r));
+                        const uint32_t mine = pack_bf16(div_by(num[hh][c], by[hh], r), div_by(num[hh][c + 1], by[hh], r));
                         const uint32_t other = (uint32_t)dpp_i<DPP_XOR1>((int)mine);
                         to[8 * c] = __builtin_amdgcn_perm(other, mine, pick);
                     }
