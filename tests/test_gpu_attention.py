@@ -337,23 +337,26 @@ def test_persistent_rows(heads):
     compare(live_case, out[:live], lse[:live], 1, rows=rows, tag=f"persistent heads {heads}")
 
 
-@pytest.mark.parametrize("ratio,lengths,heads", [
-    (128, [20000, 40, 1], 8),    # tiled rows of 151-156 compressed rows, short rows, a keyless row
-    (128, [16990, 300, 1], 8),   # rows of 128 compressed rows (joint) and of 129-132 (tiled) in one chunk
-    (128, [3000, 140, 1], 8),    # joint rows (1-23 compressed rows) and window-only rows (position < 127)
-    (128, [20000, 40, 1], 12),   # two rows per token, no residual codes: tiled
-    (1, [3000, 40, 1], 8),       # window-only cache
-    (1, [3000, 40, 1], 12),      # window-only, two rows per token (c8_rows head groups)
+@pytest.mark.parametrize("ratio,lengths,heads,chunk", [
+    (128, [20000, 40, 1], 8, 600),    # tiled rows of 151-156 compressed rows, short rows, a keyless row
+    (128, [16990, 300, 1], 8, 600),   # rows of 128 compressed rows (joint) and of 129-132 (tiled) in one chunk
+    (128, [3000, 140, 1], 8, 600),    # joint rows (1-23 compressed rows) and window-only rows (position < 127)
+    (128, [20000, 40, 1], 12, 600),   # 1238 rows, two per token, no residual codes: octets (c8_chunk)
+    (128, [20000, 40, 1], 12, 200),   # 438 of them: one work-group per row (c8_attention head groups)
+    (1, [3000, 40, 1], 8, 600),       # window-only cache
+    (1, [3000, 40, 1], 12, 600),      # window-only, 1238 rows: octets (c8_chunk)
+    (1, [3000, 40, 1], 12, 200),      # and 438: rows of sixteen heads (c8_rows)
 ])
-def test_persistent_dense_rows(ratio, lengths, heads):
+def test_persistent_dense_rows(ratio, lengths, heads, chunk):
     """One-partition C128 and window-only launches of more rows than CUs:
     window-only launches run c8_rows (two four-wave work-groups per CU taking
-    rows in turn), C128 launches one work-group per row, rows of 1-128
-    compressed rows being joint rows.  Bit-exact with the checker's plan for
-    the launch (joint_dense per row at one partition), with graph-padding
-    rows and a keyless row as in the C4 case."""
+    rows in turn), C128 launches one work-group per row, and both c8_chunk
+    (eight rows to a work-group) from about a thousand rows of eight heads on.
+    C128 rows of 1-128 compressed rows are joint rows.  Bit-exact with the
+    checker's plan for the launch (joint_dense per row at one partition), with
+    graph-padding rows and a keyless row as in the C4 case."""
     from npu_sparse_attn_sharedkv_int8 import c8_attention
-    case = workloads.make_case(82, ratio, [600, 5, 2], lengths, heads=heads)
+    case = workloads.make_case(82, ratio, [chunk, 5, 2], lengths, heads=heads)
     pad = 12
     live = int(case["cu_q"][-1])
     case["q"] = np.concatenate([case["q"], np.full((pad, heads, 512), 0x7FC0, np.uint16)])
