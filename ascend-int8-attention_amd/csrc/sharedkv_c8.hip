@@ -1684,7 +1684,7 @@ __device__ __forceinline__ Request find_request(global_i32 cu, global_i32 lens, 
 // memory.  Each wave takes 32 keys in QK (the rows it copied: no barrier
 // before it) and 128 output columns in PV.
 // Bound by instruction issue: 391 VALU instructions a wave and tile (most of
-// them the FP32 sequence), VALU 58 % and LDS 42 % busy; with every row an L2
+// them the FP32 sequence), VALU 57 % and LDS 41 % busy; with every row an L2
 // hit a prefill chunk takes the same time.  Eight waves a work-group at 128
 // VGPRs were slower (130 against 116 us on the chunk below).
 // Measured on MI355X, LDS DMA copies and rows of eight heads -> this: decode
@@ -1701,8 +1701,8 @@ __device__ __forceinline__ Request find_request(global_i32 cu, global_i32 lens, 
 // RATIO 4: the window tile and up to eight compressed tiles, every row's HBM
 // address resident in LDS.  RATIO 1: the window tile alone.  (C128 launches
 // run c8_chunk or c8_attention.)  No explicit original slots.  STREAM:
-// non-temporal KV loads (decode-shaped launches).  ANYH: any head count up
-// to eight.
+// non-temporal KV loads (decode-shaped launches).  ANYH: any head count, up
+// to eight without WIDE.
 // When graph padding leaves fewer live rows than the launch's capacity and
 // the launch may merge (`fused`: partition states and tickets supplied), the
 // live rows are re-planned with c8_attention's PLAN_FEW / PLAN_MANY rule
@@ -3039,7 +3039,7 @@ c8_pairs(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
 // Bound by the FP32 sequence (about 1250 VALU instructions a wave and tile,
 // 4.2 us for the two waves of a SIMD) and the LDS reads (1 MiB a tile and
 // work-group, 3.4 us), which overlap only in part: a tile takes about 6 us, a
-// window-only octet about 15.  Three requests of 662 C128 rows: VALU 72 %, LDS
+// window-only octet about 15.  Three requests of 662 C128 rows: VALU 68 %, LDS
 // 24 % busy.  Measured on MI355X, before -> after: B = 1 x T = 2048, C128 at
 // 8 K / 32 K / 128 K context 62 / 79 / 160 -> 27 / 33 / 68 us, window-only
 // 26 -> 17.5; T = 4096 C128 at 32 K 156 -> 62, window-only 48 -> 31.
@@ -3234,7 +3234,7 @@ c8_chunk(const uint64_t cu_q, const uint64_t seq_lens, const uint64_t q_base, co
     // Work-groups that would have nothing to do in the last round of octets
     // take the tails, one each, if they suffice or an octet is crowded (then
     // further rounds take the rest).  Otherwise an octet takes its two
-    // requests at once (`pairs`, below).
+    // requests at once (`two`, below).
     // Tails of at most SHORT_TAIL rows (decode requests beside prefill chunks)
     // are taken whole.
     auto inside = [&](int c0) { return c0 * HG % CHUNK_ROWS != 0; };
